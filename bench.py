@@ -591,6 +591,7 @@ def stream_main(args) -> int:
         for key in ("launches", "kernelMs", "localLaunches", "localKernelMs"):
             prof[key] = timed[key]
         progress("work counters collected")
+    repeated_iterations, repeated = ctx.skipped()
     ctx.set_profiling(0)
     tuning = ctx.tuning()
     ctx.close()
@@ -614,6 +615,9 @@ def stream_main(args) -> int:
                    "updates_per_step": updates},
         "batch_latency_ms": {"p50": float(np.percentile(lat, 50)),
                              "p99": float(np.percentile(lat, 99))},
+        # counted in value, and not run: iterations that repeat an earlier state
+        "repeated": {"iterations_per_step": repeated_iterations, "updates_per_step": repeated,
+                     "run_updates_per_s": (updates - repeated) / wall},
         "tuning": tuning,
         "batches": [{k: s[k] for k in ("iterations", "updates", "frontier0", "numSubEdges",
                                        "numComponents", "timeMs", "accuracy")} for s in stats],
@@ -623,8 +627,8 @@ def stream_main(args) -> int:
                                 "local_launches": timed["localLaunches"]},
     }
     if prof is not None:
-        out["propagation_kernels"] = add_random_access(engine_rooflines(prof, updates), prof,
-                                                       updates, N, out)
+        out["propagation_kernels"] = add_random_access(
+            engine_rooflines(prof, updates - repeated), prof, updates - repeated, N, out)
     if args.calibrate_copy_mib > 0:
         out["copy_calibration"] = copy_calibration(args.calibrate_copy_mib)
     print(json.dumps(out))
@@ -855,6 +859,7 @@ def main() -> int:
     ctx.run_all()
     ctx.synchronize()
     work = ctx.prop_profile()
+    repeated_iterations, repeated = ctx.skipped()
     ctx.set_profiling(0)
     ctx.close()
     prof = dict(work)
@@ -863,9 +868,10 @@ def main() -> int:
 
     ms_per_step = 1000.0 * wall / args.steps
     value = updates / (wall / args.steps)
-    engines = engine_rooflines(prof, updates)
+    run = updates - repeated  # updates the kernels ran: what their bytes and rates count
+    engines = engine_rooflines(prof, run)
     ra_out = {}
-    engines = add_random_access(engines, prof, updates, args.nodes, ra_out)
+    engines = add_random_access(engines, prof, run, args.nodes, ra_out)
     dominant = max(engines, key=lambda k: engines[k]["kernel_ms_per_step"])
     dom = engines[dominant]
     achieved = dom["achieved_gbs"]
@@ -889,6 +895,12 @@ def main() -> int:
                    "updates_per_step": updates},
         "batch_latency_ms": {"p50": float(np.percentile(lat, 50)),
                              "p99": float(np.percentile(lat, 99))},
+        # of updates_per_step, those of iterations that repeat an earlier
+        # state bit for bit (a batch alternating between two states until the
+        # iteration cap): they are counted, and not run; value counts them,
+        # run_updates_per_s does not
+        "repeated": {"iterations_per_step": repeated_iterations, "updates_per_step": repeated,
+                     "run_updates_per_s": run / (wall / args.steps)},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic(dominant) if args.nodes == 500000 else None,

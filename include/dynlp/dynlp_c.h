@@ -290,6 +290,14 @@ int dlp_context_run_batch(dlp_context *ctx, int b);
 /* reset + every batch. */
 int dlp_context_run_all(dlp_context *ctx);
 int dlp_context_synchronize(dlp_context *ctx);
+/* Iterations of the batches since the last reset, and the sum of their
+ * frontier sizes, that were counted (iterations / updates of the batch
+ * stats) without being run, because the propagation had come back to the
+ * state of two iterations before bit for bit and would have alternated
+ * between two states until maxIterations (synchronises; no counterpart in
+ * the reference, which runs them).  0 while a trace records every
+ * iteration's frontier size. */
+int dlp_context_skipped(dlp_context *ctx, int64_t *iterations, int64_t *updates);
 /* Copies the current labels (N floats) to host. */
 int dlp_context_read_labels(dlp_context *ctx, float *labels);
 /* Stats of batch b from the most recent run (synchronises). */

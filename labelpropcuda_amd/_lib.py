@@ -238,6 +238,7 @@ SIGNATURES = {
     "dlp_context_run_batch": (C.c_int, [_VP, C.c_int]),
     "dlp_context_run_all": (C.c_int, [_VP]),
     "dlp_context_synchronize": (C.c_int, [_VP]),
+    "dlp_context_skipped": (C.c_int, [_VP, i64p, i64p]),
     "dlp_context_read_labels": (C.c_int, [_VP, f32p]),
     "dlp_context_batch_stats": (C.c_int, [_VP, C.c_int, C.POINTER(BatchStats)]),
     "dlp_context_set_trace": (C.c_int, [_VP, C.POINTER(Trace)]),

@@ -76,6 +76,11 @@ struct DevCounters {
    * from the vertices each batch changes (zeroed by a reset only) */
   unsigned long long accCorrect;
   unsigned long long accTotal;
+  /* iterations, and the sum of their frontier sizes, that repeated an
+   * earlier state bit for bit and were counted without being run (since the
+   * last reset) */
+  unsigned long long skippedIterations;
+  unsigned long long skippedUpdates;
 };
 
 /* exit reasons of the LDS-resident propagation kernel */

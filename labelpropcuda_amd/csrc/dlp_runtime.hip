@@ -923,6 +923,7 @@ PropArgs dlp_ctx_prop_args(const dlp_context *c) {
    * (holes for this batch's deletions on both sides), so it is symmetric
    * when the full graph is */
   a.symmetric = c->symmetric ? 1 : 0;
+  a.cycles = a.iterSizes ? 0 : 1;
   return a;
 }
 
@@ -1001,6 +1002,19 @@ extern "C" int dlp_context_synchronize(dlp_context *c) {
     return DLP_ERR_STATE;
   }
   DLP_HIP(hipStreamSynchronize(c->stream));
+  return DLP_OK;
+}
+
+extern "C" int dlp_context_skipped(dlp_context *c, int64_t *iterations, int64_t *updates) {
+  if (!c || !iterations || !updates) {
+    dlp_set_error_("dlp_context_skipped: NULL argument");
+    return DLP_ERR_INVALID;
+  }
+  DLP_HIP(hipStreamSynchronize(c->stream));
+  DevCounters ctr;
+  DLP_HIP(hipMemcpy(&ctr, c->d.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
+  *iterations = (int64_t)ctr.skippedIterations;
+  *updates = (int64_t)ctr.skippedUpdates;
   return DLP_OK;
 }
 

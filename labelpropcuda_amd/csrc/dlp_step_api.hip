@@ -329,6 +329,7 @@ int propagate_on(const PropScratch &ps, const int *rowPtr, const int *colInd, co
   a.iterSizes = nullptr;
   a.iterSizesCap = 0;
   a.profile = 0;
+  a.cycles = 1;
   a.delta = delta;
   a.waveRowMin = kDefaultWaveRowMin;
   a.blockRowMin = kDefaultBlockRowMin;

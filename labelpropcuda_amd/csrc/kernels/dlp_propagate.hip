@@ -410,6 +410,8 @@ __device__ int block_scan_lds(const int *a, int *out, int n, int *tmp /* >= 17 i
 enum {
   SH_GEN, SH_CC, SH_NCAND, SH_NCORE, SH_BIG, SH_REBUILD, SH_NOVF, SH_HASLONG,
   SH_NHE, SH_NHI, SH_QC0, SH_QC1, SH_QC2, SH_NLONG0, SH_NLONG1, SH_INELIG, SH_MAXLEN,
+  SH_LASTACT, /* last iteration that changed a label bit, or whose frontier
+                 differs from the one two before (owner mode) */
   SH_COUNT
 };
 
@@ -524,6 +526,16 @@ __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
   }
 }
 
+__device__ __forceinline__ bool same_bits(float x, float y) {
+  return __float_as_int(x) == __float_as_int(y);
+}
+
+/* counts the iterations a cycle lets the caller pass over (one thread) */
+__device__ __forceinline__ void count_skipped(DevCounters *c, int skip, unsigned long long sum) {
+  c->skippedIterations += (unsigned long long)skip;
+  c->skippedUpdates += sum;
+}
+
 /* rlL word of a core vertex: row length, and a flag for rows that name an
  * eligible vertex outside the core */
 constexpr int kRowLenMask = 0x3fffffff;
@@ -545,8 +557,9 @@ struct LocalShared {
   int ownerCount;     /* queue rebuilt from the owner-mode flags */
   unsigned long long ownerSum; /* frontier sizes of the owner-mode iterations */
   /* register-mask owner mode with several waves: per wave and iteration
-   * parity, the changed-vertex mask, whether a mark left the core, and the
-   * size of the wave's next frontier */
+   * parity, the changed-vertex mask, whether a mark left the core (bit 0) and
+   * whether a label bit or the frontier changed (bit 1), and the size of the
+   * wave's next frontier */
   unsigned long long xChanged[2][kMaskWavesMax];
   unsigned char xOut[2][kMaskWavesMax];
   unsigned char xCount[2][kMaskWavesMax]; /* 0 .. 64 */
@@ -679,12 +692,15 @@ __device__ __forceinline__ int owner_iterations(
   float l0[V], l1[V];
   int len[V], ro[V];
   bool own[V], hasOut[V], entered[V];
+  unsigned hist[V]; /* flags of the last iteration (bit 0) and the one before */
+  int nPrev = 0;    /* size of the last iteration's frontier */
 #pragma unroll
   for (int v = 0; v < V; ++v) {
     const int ci = tid + v * LT;
     own[v] = ci < nCore;
     len[v] = ro[v] = 0;
     hasOut[v] = entered[v] = false;
+    hist[v] = 0u;
     l0[v] = l1[v] = 0.0f;
     if (own[v]) {
       const int rl = rlL[ci];
@@ -724,8 +740,11 @@ __device__ __forceinline__ int owner_iterations(
     if (tid == 0) sh[SH_QC0 + (k + 1) % 3] = 0;
     const LocalIter it{stampL, nullptr, nullptr, sh, haloE, nullptr, dumOut, nCore, nHE,
                        k + 1, stampBase + k + 1, stampBase};
+    bool act = false; /* a label bit changed, or the flag of two iterations ago differs */
 #pragma unroll
     for (int v = 0; v < V; ++v) {
+      act = act || (f[v] ? 1u : 0u) != (hist[v] >> 1);
+      hist[v] = ((hist[v] << 1) & 2u) | (f[v] ? 1u : 0u);
       if (!__any(f[v])) continue;  // wave-uniform
       const int ci = own[v] ? tid + v * LT : 0;
       const float oldLabel = kb ? l1[v] : l0[v];
@@ -747,6 +766,7 @@ __device__ __forceinline__ int owner_iterations(
           owner_rows<kLaneRowMax, true>(a, l, it, len[v] <= SR ? rowS : recL + ro[v], nullSlot,
                                         Fo, Fn, nxt, dumOut, lanePath, ci, len[v], hasOut[v],
                                         oldLabel, nl, changed, prof);
+        act = act || (lanePath && !same_bits(nl, kb ? l0[v] : l1[v]));
         l0[v] = (lanePath && kb) ? nl : l0[v];
         l1[v] = (lanePath && !kb) ? nl : l1[v];
       }
@@ -772,6 +792,7 @@ __device__ __forceinline__ int owner_iterations(
         lnl = __shfl(lnl, 0, 64);
         changed = __shfl(changed, 0, 64);
         if (lane == src) {
+          act = act || !same_bits(lnl, kb ? l0[v] : l1[v]);
           if (kb)
             l0[v] = lnl;
           else
@@ -795,8 +816,14 @@ __device__ __forceinline__ int owner_iterations(
       *(f[v] ? &cur[ci] : dumOut) = 0;
       entered[v] = entered[v] || (f[v] && k > kBuild);
     }
+    if (__any(act) && lane == 0) sh[SH_LASTACT] = k;
     __syncthreads();
     const int n = sh[SH_QC0 + k % 3];
+    /* the last iterations k-2 .. k left no trace: the state of k is that of
+     * k - 2.  A wave already in iteration k + 1 may have stored k + 1, but
+     * only after it found no cycle here, from a value that every wave finds
+     * no cycle from. */
+    const bool cycle = a.cycles && sh[SH_LASTACT] < k - 2;
     if (n == 0) {  // uniform
       reason = DLP_LOCAL_CONVERGED;
       break;
@@ -808,6 +835,20 @@ __device__ __forceinline__ int owner_iterations(
     }
     ++k;
     if (sh[SH_REBUILD]) break;  // uniform after the barrier
+    const int skip = cycle ? dlp_cycle_skip(k, maxIter) : 0;
+    if (skip > 0) {     // uniform: frontiers nPrev, n, nPrev, n, ... up to the cap
+      __syncthreads();  // every wave has read its counts
+      if (tid == 0) {
+        const unsigned long long sum =
+            (unsigned long long)(skip / 2) * (unsigned long long)(nPrev + n);
+        passUpdates += sum;
+        count_skipped(c, skip, sum);
+        sh[SH_QC0] = sh[SH_QC0 + 1] = sh[SH_QC0 + 2] = 0;
+      }
+      k += skip;
+      __syncthreads();
+    }
+    nPrev = n;
   }
 
   /* flags of iteration k -> its queue; stamps of the vertices that entered */
@@ -949,11 +990,15 @@ __device__ __forceinline__ int wave_owner_iterations(
   unsigned outPos[V]; /* row positions naming eligible vertices outside the core */
   float Wr[V];        /* weight sums of the rows */
   bool entered[V];
+  unsigned long long fm1[V]; /* frontier of the last iteration */
+  int quiet = 0;             /* iterations since a label bit changed */
+  int nPrev = 0;             /* size of the last iteration's frontier */
 #pragma unroll
   for (int r = 0; r < V; ++r) {
     const int ci = lane + 64 * r;
     const bool own = ci < nCore;
     ownMask[r] = dlp_ballot(own);
+    fm1[r] = 0ull;
     entered[r] = false;
     fm[r] = dlp_ballot(own && flags0[ci] != 0);
     len[r] = own ? (rlL[ci] & kRowLenMask) : 0;
@@ -997,12 +1042,13 @@ __device__ __forceinline__ int wave_owner_iterations(
     const float *Fo = kb ? lab1L : lab0L;
     float *Fn = kb ? lab0L : lab1L;
     unsigned long long cm[V];
-    bool ch[V], anyOut = false;
+    bool ch[V], anyOut = false, diff = false;
 #pragma unroll
     for (int r = 0; r < V; ++r) {
       const bool f = (fm[r] >> lane) & 1ull;
       const float old = kb ? l1[r] : l0[r];
       const float nl = mask_row_label_any<L>(src[r], w[r], Wr[r], Fo, nullSlot, f, len[r], old);
+      diff = diff || (f && !same_bits(nl, kb ? l0[r] : l1[r]));
       ch[r] = f && fabsf(nl - old) > a.delta;
       *(f ? &Fn[lane + 64 * r] : (float *)dumOut) = nl;
       l0[r] = (f && kb) ? nl : l0[r];
@@ -1025,8 +1071,12 @@ __device__ __forceinline__ int wave_owner_iterations(
           if ((outPos[r] >> p) & 1u) prof.A += mark_outside(a, l, it, haloE[src[r][p] - nCore]);
       }
     }
+    quiet = __any(diff) ? 0 : quiet + 1;  // uniform
     /* next frontier: every changed vertex and the core vertices their rows
      * name */
+    unsigned long long fm0[V]; /* frontier k */
+#pragma unroll
+    for (int r = 0; r < V; ++r) fm0[r] = fm[r];
     if (symmetric) {
 #pragma unroll
       for (int r = 0; r < V; ++r) {
@@ -1052,6 +1102,26 @@ __device__ __forceinline__ int wave_owner_iterations(
     ++k;
     __syncthreads();  // new labels (and mark_outside's writes) visible to every lane
     if (rebuild) break;
+    /* no label bit changed in the last two iterations and their frontiers
+     * return: the state of iteration k is that of k - 2 */
+    if (a.cycles && quiet >= 2) {  // uniform
+      bool same = true;
+#pragma unroll
+      for (int r = 0; r < V; ++r) same = same && fm[r] == fm1[r];
+      const int skip = same ? dlp_cycle_skip(k, maxIter) : 0;
+      if (skip > 0) {  // frontiers nPrev, n, nPrev, n, ... up to the cap
+        const unsigned long long sum =
+            (unsigned long long)(skip / 2) * (unsigned long long)(nPrev + n);
+        if (lane == 0) {
+          passUpdates += sum;
+          count_skipped(c, skip, sum);
+        }
+        k += skip;
+      }
+    }
+    nPrev = n;
+#pragma unroll
+    for (int r = 0; r < V; ++r) fm1[r] = fm0[r];
   }
 
   /* the masks of iteration k -> its queue (by core index); stamps of the
@@ -1146,7 +1216,12 @@ __device__ __forceinline__ int mask_owner_iterations(
     }
   }
   const float Wrow = mask_row_weight<L>(w);
+  unsigned long long fm1 = 0ull, fm2 = 0ull; /* frontiers of the last iteration and the
+                                                one before */
+  int quiet = 0; /* iterations since a label bit changed or a frontier differed from
+                    the one two before */
   int n = nq;  // size of frontier k, known for the first iteration
+  int nPrev = 0; /* size of frontier k - 1 */
   __syncthreads();  // the flags are read
 
   int reason = 0;
@@ -1172,6 +1247,9 @@ __device__ __forceinline__ int mask_owner_iterations(
     if (fm != 0ull)  // wave-uniform: a wave with no flagged vertex only syncs
       nl = mask_row_label_any<L>(src, w, Wrow, Fo, nullSlot, f, len, old);
     const bool ch = f && fabsf(nl - old) > a.delta;
+    const bool actW = __any(f && !same_bits(nl, kb ? l0 : l1)) || fm != fm2;
+    fm2 = fm1;
+    fm1 = fm;
     *(f ? &Fn[tid] : (float *)dumOut) = nl;
     l0 = (f && kb) ? nl : l0;
     l1 = (f && !kb) ? nl : l1;
@@ -1188,9 +1266,10 @@ __device__ __forceinline__ int mask_owner_iterations(
     }
     if (lane == 0) {
       S.xChanged[kb][wave] = cmW;
-      S.xOut[kb][wave] = outW ? 1u : 0u;
+      S.xOut[kb][wave] = (outW ? 1u : 0u) | (actW ? 2u : 0u);
     }
     __syncthreads();
+    nPrev = n;
     if (!first) {  // the size of frontier k, published in iteration k - 1
       int cnt[W];
 #pragma unroll
@@ -1216,7 +1295,8 @@ __device__ __forceinline__ int mask_owner_iterations(
     for (int q = 0; q < W; ++q) xc[q] = S.xChanged[kb][q];
 #pragma unroll
     for (int q = 0; q < W; ++q) meet |= out[q] & xc[q];
-    const bool rebuild = outs != 0;
+    const bool rebuild = (outs & 1) != 0;
+    quiet = (outs & 2) ? 0 : quiet + 1;
     fm = dlp_ballot(ch || meet != 0ull) & ownMask;
     if (lane == 0) S.xCount[kb][wave] = (unsigned char)__popcll(fm);
     if (tid == 0) {
@@ -1226,6 +1306,18 @@ __device__ __forceinline__ int mask_owner_iterations(
     ownerSum += (unsigned long long)n;
     ++k;
     if (rebuild) break;  // uniform
+    /* iterations k-3 .. k-1 left no trace: the state of k-1 is that of k-3,
+     * and so is that of k the one of k-2 */
+    const int skip = (a.cycles && quiet >= 3) ? dlp_cycle_skip(k, maxIter) : 0;
+    if (skip > 0) {  // uniform: frontiers nPrev, n, nPrev, n, ... up to the cap
+      const unsigned long long sum =
+          (unsigned long long)(skip / 2) * (unsigned long long)(nPrev + n);
+      if (tid == 0) {
+        passUpdates += sum;
+        count_skipped(c, skip, sum);
+      }
+      k += skip;
+    }
   }
 
   /* the masks of iteration k -> its queue (by core index); stamps of the
@@ -1340,6 +1432,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       sh[SH_NLONG0] = 0;
       sh[SH_NLONG1] = 0;
       sh[SH_INELIG] = 0;
+      sh[SH_LASTACT] = k;
     }
     __syncthreads();
     const int gen = sh[SH_GEN], cc = sh[SH_CC], nCand = sh[SH_NCAND];

@@ -432,6 +432,13 @@ class Context:
     def synchronize(self):
         check(self._lib.dlp_context_synchronize(self._h))
 
+    def skipped(self):
+        """(iterations, updates) since the last reset that repeated an earlier
+        state bit for bit and were counted without being run."""
+        it, up = C.c_int64(), C.c_int64()
+        check(self._lib.dlp_context_skipped(self._h, C.byref(it), C.byref(up)))
+        return it.value, up.value
+
     def labels(self) -> np.ndarray:
         out = np.zeros(self.inputs.numNodes, np.float32)
         check(self._lib.dlp_context_read_labels(self._h, _ptr(out, C.c_float)))

@@ -1,0 +1,127 @@
+"""Batches that run into the iteration cap alternate between two states: the
+propagation kernels count the iterations that repeat the state of two
+iterations before bit for bit instead of running them.  Labels, iteration and
+update counts must stay the oracle's, which runs every one of them, for every
+engine and for an even and an odd number of iterations left."""
+import numpy as np
+import pytest
+
+import labelpropcuda_amd as L
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.int32)
+
+
+def from_rows(rows, labels, prefix, batches):
+    """Inputs of a graph given as {neighbour: weight} rows, through the graph
+    text files and the reference batch generator."""
+    rows = [sorted(r.items()) for r in rows]
+    for name, vals in (("RowPtr", np.cumsum([0] + [len(r) for r in rows])),
+                       ("ColInd", [v for r in rows for v, _ in r]),
+                       ("Values", [f"{w:.6f}" for r in rows for _, w in r]),
+                       ("TrueLabels", [f"{i} {c}" for i, c in enumerate(labels)])):
+        with open(prefix + name + ".txt", "w") as f:
+            f.write("\n".join(map(str, vals)) + "\n")
+    return L.dynlp.from_graph_files(prefix, batches, 42)
+
+
+def star_tree(prefix, hubs=40, leaves=30, seed=2, batches=6):
+    """A random tree of hubs, each with about `leaves` leaves: deletions
+    detach bipartite subtrees, whose labels alternate; the hubs' rows are
+    longer than one lane sums."""
+    rng = np.random.default_rng(seed)
+    n = hubs * (leaves + 1)
+    ids = rng.permutation(n)
+    rows = [{} for _ in range(n)]
+    for x in range(1, n):
+        u, v = int(ids[x]), int(ids[rng.integers(min(x, hubs))])
+        rows[u][v] = rows[v][u] = float(rng.uniform(0.05, 1.0))
+    return from_rows(rows, rng.permutation(np.arange(n) % 2), prefix, batches)
+
+
+def one_sided(inp, prefix, share=0.1, seed=2):
+    """`inp`'s graph with a share of its entries dropped on one side."""
+    rng = np.random.default_rng(seed)
+    rows = [{int(v): float(w) for v, w in zip(inp.colInd[a:b], inp.values[a:b])
+             if rng.random() >= share}
+            for a, b in zip(inp.rowPtr[:-1], inp.rowPtr[1:])]
+    return from_rows(rows, inp.trueLabels.astype(int), prefix, 8)
+
+
+_ORACLE = {}
+
+
+def oracle_run(key, inp, cap):
+    """(labels bits, iterations, updates) after every batch."""
+    if (key, cap) not in _ORACLE:
+        orc = Oracle(inp, maxIterations=cap)
+        res = []
+        for b in range(inp.numBatches):
+            orc.run_batch(b)
+            st = orc.stats()
+            res.append((bits(orc.labels()).copy(), st["iterations"], st["updates"]))
+        assert any(r[1] == cap for r in res), "no batch reaches the cap"
+        _ORACLE[key, cap] = res
+    return _ORACLE[key, cap]
+
+
+def graph(kind, tmp_path):
+    if kind == "random":
+        return L.generate(5000, 5, 6, 42)
+    if kind == "sparse":
+        return L.generate(2000, 3, 8, 3)
+    if kind == "long rows":
+        return star_tree(str(tmp_path / "star_"))
+    return one_sided(L.generate(2000, 3, 8, 3), str(tmp_path / "one_"))
+
+
+def check(kind, inp, cap, skips=True, **tuning):
+    want = oracle_run(kind, inp, cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        ctx.set_tuning(**tuning)
+        for _ in range(2):  # the second pass starts from the first one's device state
+            ctx.reset()
+            for b in range(inp.numBatches):
+                ctx.run_batch(b)
+                st = ctx.stats(b)
+                assert (st["iterations"], st["updates"]) == want[b][1:], f"batch {b}"
+                assert np.array_equal(bits(ctx.labels()), want[b][0]), f"batch {b}: labels"
+        it, up = ctx.skipped()
+        if skips:
+            assert 0 < it < sum(r[1] for r in want) and 0 < up < sum(r[2] for r in want)
+
+
+CAPS = [20000, 20001]
+
+
+@pytest.mark.parametrize("cap", CAPS)
+@pytest.mark.parametrize("kind,tuning", [
+    ("random", dict()),                                       # register-mask kernels
+    ("random", dict(localOwnerAfter=1)),
+    ("random", dict(localOwnerAfter=1, maskOwnerMax=-1)),     # flags, one vertex per thread
+    ("random", dict(localOwnerAfter=1, maskOwnerMax=-1, localShape=4)),  # several per thread
+    ("sparse", dict(localOwnerAfter=1)),
+    ("long rows", dict(localOwnerAfter=1)),                   # rows summed by a wave
+    ("one-sided", dict(localOwnerAfter=1)),                   # one wave, rows OR-reduced
+])
+def test_owner_kernels(gpu_available, tmp_path, kind, tuning, cap):
+    check(kind, graph(kind, tmp_path), cap, **tuning)
+
+
+def test_trace_runs_every_iteration(gpu_available):
+    """A trace records every iteration's frontier size, so nothing is passed
+    over while one is on."""
+    inp, cap = L.generate(5000, 5, 4, 42), 6000
+    orc = Oracle(inp, maxIterations=cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        tr = ctx.enable_trace(maxFrontierSizes=cap)
+        ctx.reset()
+        for b in range(inp.numBatches):
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            assert np.array_equal(tr.snapshot()["frontierSizes"], orc.frontier_sizes())
+        assert ctx.skipped() == (0, 0)
