@@ -62,7 +62,9 @@ struct PropArgs {
  * stopped changing after 5,268 iterations at the median, 54,559 at most.
  * Whole streams of ten batches, one pass: 5,000 vertices 165.1 -> 48.3 ms,
  * 50,000 vertices 395.6 -> 139.3 ms, 500,000 vertices 543.6 -> 206.5 ms with
- * the test in the owner-mode LDS kernels. */
+ * the test in the owner-mode LDS kernels; with it in the queue iterations of
+ * the shared launch, 40 graphs of 2,000 to 16,000 vertices (8 batches each)
+ * 1,434 -> 770 ms. */
 __host__ __device__ inline int dlp_cycle_skip(int k, int maxIter) { return (maxIter - k) & ~1; }
 constexpr int kDefaultWaveRowMin = 64;
 constexpr int kDefaultBlockRowMin = 1024;

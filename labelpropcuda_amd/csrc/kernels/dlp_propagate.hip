@@ -412,12 +412,22 @@ enum {
   SH_NHE, SH_NHI, SH_QC0, SH_QC1, SH_QC2, SH_NLONG0, SH_NLONG1, SH_INELIG, SH_MAXLEN,
   SH_LASTACT, /* last iteration that changed a label bit, or whose frontier
                  differs from the one two before (owner mode) */
+  SH_LASTDIFF, /* queue iterations: the last one that changed a label bit,   */
+  SH_LASTMISS, /* and the last one whose next frontier is not known to be
+                  made of vertices of the frontier two before it             */
   SH_COUNT
 };
 
+__device__ __forceinline__ bool same_bits(float x, float y) {
+  return __float_as_int(x) == __float_as_int(y);
+}
+
+/* LDS stamp of a core vertex that entered no frontier in the pass */
+constexpr int kNoStamp = -4;
+
 /* state of one local iteration shared by its row paths */
 struct LocalIter {
-  int *stampL;
+  int *stampL;       /* stamps of the next frontier (one array per parity)   */
   int *qout;
   int *qcOut;
   int *sh;
@@ -448,13 +458,16 @@ __device__ __forceinline__ unsigned mark_outside(const PropArgs &a, const LocalA
  * writes are branch-free: a lane with nothing to mark or write at a
  * position targets its own dummy LDS word (a stamp that stays INT_MAX, a
  * scratch slot), so a lane waits for a few LDS round trips, not one per
- * entry, and no exec-mask juggling is needed. */
-template <int L, bool MASKED>
+ * entry, and no exec-mask juggling is needed.  With CYC, `diff` is set when a
+ * label bit changes and, if `watch` (uniform), `miss` when a vertex enters
+ * the next frontier that was not in the frontier two before it (its stamp of
+ * that parity). */
+template <int L, bool MASKED, bool CYC>
 __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
                                           const LocalIter &it, const int2 *row, int nullSlot,
                                           const float *Fo, float *Fn, bool act, int ci, int len,
-                                          bool hasOut, unsigned &profE, unsigned &profC,
-                                          unsigned &profA) {
+                                          bool hasOut, bool watch, bool &diff, bool &miss,
+                                          unsigned &profE, unsigned &profC, unsigned &profA) {
   static_assert(L + 1 <= 32, "hit mask is 32 bits");
   int tt[L];
   float ww[L], ff[L];
@@ -468,6 +481,7 @@ __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
 #pragma unroll
   for (int j = 0; j < L; ++j) ff[j] = Fo[tt[j]];
   const float oldLabel = Fo[ci];
+  const float cur = CYC ? Fn[ci] : 0.0f; /* the label that nl replaces */
   float W, S;
   dlp::lane_row_sums<L>(
       L,
@@ -478,6 +492,7 @@ __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
       W, S);
   const float nl = dlp::new_label(W, S, oldLabel);
   const bool changed = act && fabsf(nl - oldLabel) > a.delta;
+  if (CYC) diff = diff || (act && !same_bits(nl, cur));
   if (act) {
     Fn[ci] = nl;
     profE += (unsigned)len;
@@ -496,6 +511,10 @@ __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
   unsigned hit = 0u;
 #pragma unroll
   for (int j = 0; j <= L; ++j) hit |= (olds[j] < next ? 1u : 0u) << j;
+  if (CYC && watch) {  // uniform
+#pragma unroll
+    for (int j = 0; j <= L; ++j) miss = miss || (olds[j] < next && olds[j] != next - 2);
+  }
   /* eligible vertices outside the core (rows flagged at the build) */
   if (__any(changed && hasOut)) {  // wave-uniform
     if (changed && hasOut) {
@@ -524,10 +543,6 @@ __device__ __forceinline__ void lane_rows(const PropArgs &a, const LocalArgs &l,
       pos += h ? 1 : 0;
     }
   }
-}
-
-__device__ __forceinline__ bool same_bits(float x, float y) {
-  return __float_as_int(x) == __float_as_int(y);
 }
 
 /* counts the iterations a cycle lets the caller pass over (one thread) */
@@ -1385,11 +1400,18 @@ __device__ __forceinline__ int wave_owner_dispatch(
 
 /* Runs LDS-resident passes from iteration k (updated) until the frontier
  * empties, k reaches maxIter, or the working set outgrows the LDS budget;
- * returns the DLP_LOCAL_* reason.  All LT threads of the work-group call
+ * returns the DLP_LOCAL_* reason.  capIter is the batch's iteration cap, up
+ * to which a cycle is passed over (k may then end above maxIter).  CYC:
+ * queue iterations look for cycles too (dlp_cycle_skip).  The shared launch
+ * of many graphs needs it, its graphs stay in queue iterations; the
+ * single-graph queue kernel hands a long-lived frontier to owner mode after
+ * 1,024 iterations, and the test would cost it 12 spilled registers.  All LT threads of the work-group call
  * it; `pool` is the dynamic LDS (l.ldsWords words). */
-template <int LT, int SR, bool OWNER, bool MASK = false>
+template <int LT, int SR, bool OWNER, bool MASK, bool CYC>
 __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &l, int &k, int maxIter,
-                            int *pool, LocalShared &S, LocalProf &prof, int longAfter) {
+                            int capIter, int *pool, LocalShared &S, LocalProf &prof,
+                            int longAfter) {
+  static_assert(!(CYC && OWNER), "owner mode finds cycles by itself");
   static_assert(SR <= kLaneRowMax, "padded stride above the lane row limit");
   /* padded rows are SR + 1 records apart: with 2*(SR+1) words (SR a power
    * of two) the rows of neighbouring core vertices start in different LDS
@@ -1432,7 +1454,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       sh[SH_NLONG0] = 0;
       sh[SH_NLONG1] = 0;
       sh[SH_INELIG] = 0;
-      sh[SH_LASTACT] = k;
+      sh[SH_LASTACT] = sh[SH_LASTDIFF] = sh[SH_LASTMISS] = k;
     }
     __syncthreads();
     const int gen = sh[SH_GEN], cc = sh[SH_CC], nCand = sh[SH_NCAND];
@@ -1488,7 +1510,8 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
     const int nLab = nullSlot + 1;
     /* layout after gidL, rlL, rsL */
     const int offStamp = nCand + 2 * nCore;
-    const int offQ0 = offStamp + nCore, offQ1 = offQ0 + nCore, offLong = offQ1 + nCore;
+    const int offQ0 = offStamp + (CYC ? 2 : 1) * nCore;
+    const int offQ1 = offQ0 + nCore, offLong = offQ1 + nCore;
     const int offLab0 = offLong + nCore, offLab1 = offLab0 + nLab;
     const int offHalo = offLab1 + nLab;
     const int offRecS = (offHalo + nHE + 1) & ~1;                  // int2 aligned
@@ -1502,7 +1525,11 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       reason = DLP_LOCAL_TOO_BIG;
       break;
     }
+    /* the iteration a vertex last entered a frontier at; queue iterations
+     * keep one array per parity, so that the claim of a vertex for frontier
+     * k + 1 returns whether it was in frontier k - 1 */
     int *stampL = pool + offStamp;
+    int *stampOdd = CYC ? stampL + nCore : stampL;
     int *q0L = pool + offQ0;
     int *q1L = pool + offQ1;
     int *longL = pool + offLong;
@@ -1517,7 +1544,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       lab0L[i] = a.lab0[g];
       lab1L[i] = a.lab1[g];
       const bool inelig = a.iterStamp[g] == DLP_INT_MAX;
-      stampL[i] = inelig ? DLP_INT_MAX : -1;
+      stampL[i] = stampOdd[i] = inelig ? DLP_INT_MAX : kNoStamp;
       if (inelig) sh[SH_INELIG] = 1;
       const int beg = a.rowBeg[g], len = rlL[i];
       const bool shortRow = len <= SR;
@@ -1557,10 +1584,11 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
     const int nq = nCand - cc;
     {
       int *qin = (k & 1) ? q1L : q0L;
+      int *stampK = (k & 1) ? stampOdd : stampL;
       for (int i = tid; i < nq; i += LT) {
         const int idx = ld_agent(&l.coreIdx[qk[i]]);
         qin[i] = idx;
-        stampL[idx] = k;
+        stampK[idx] = k;
       }
       if (tid == 0) {
         sh[SH_QC0 + k % 3] = nq;
@@ -1612,8 +1640,37 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
                                               nullSlot, stampBase, rlL, rsL, recS, recL, stampL,
                                               q0L, q1L, lab0L, lab1L, haloE, passUpdates, prof);
     } else {  // queue iterations
+      int nPrev = -1, nPrev2 = -1; /* sizes of the last two frontiers of the pass */
       while (true) {
         const int n = sh[SH_QC0 + k % 3];
+        const int lastDiff = CYC ? sh[SH_LASTDIFF] : 0, lastMiss = CYC ? sh[SH_LASTMISS] : 0;
+        /* the last two iterations changed no label bit, and frontier k is
+         * made of the vertices of frontier k - 2 and as large: the state of
+         * k - 2.  (A wave ahead in this iteration may store k in these
+         * words, but only after it found no cycle here, from values that
+         * every wave finds no cycle from.) */
+        if (CYC && a.cycles && n > 0 && n == nPrev2 && lastDiff < k - 2 && lastMiss < k - 1) {
+          const int skip = dlp_cycle_skip(k, capIter);
+          if (skip > 0) {     // uniform: frontiers n, nPrev, n, nPrev, ... up to the cap
+            __syncthreads();  // every wave has read its counts
+            if (tid == 0) {
+              const unsigned long long sum =
+                  (unsigned long long)(skip / 2) * (unsigned long long)(n + nPrev);
+              passUpdates += sum;
+              count_skipped(c, skip, sum);
+              sh[SH_QC0] = sh[SH_QC0 + 1] = sh[SH_QC0 + 2] = 0;
+              sh[SH_QC0 + (k + skip) % 3] = n;
+            }
+            k += skip;
+            nPrev = nPrev2 = -1;
+            __syncthreads();
+            continue;
+          }
+        }
+        nPrev2 = nPrev;
+        nPrev = n;
+        const bool watch = CYC && a.cycles && lastDiff < k - 1;
+        bool diff = false, miss = !watch && tid == 0;
         if (n == 0) {
           reason = DLP_LOCAL_CONVERGED;
           break;
@@ -1639,7 +1696,8 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
         const float *Fo = kb ? lab1L : lab0L;
         float *Fn = kb ? lab0L : lab1L;
         int *nLongCtr = &sh[SH_NLONG0 + kb];
-        const LocalIter it{stampL, kb ? q0L : q1L, &sh[SH_QC0 + (k + 1) % 3], sh, haloE,
+        const LocalIter it{kb ? stampL : stampOdd, kb ? q0L : q1L, &sh[SH_QC0 + (k + 1) % 3], sh,
+                           haloE,
                            dummyStamp, dummyOut, nCore, nHE, k + 1, stampBase + k + 1,
                            stampBase};
 
@@ -1661,16 +1719,18 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
           if (__any(shortRow)) {  // wave-uniform
             const int2 *row = recS + ci * RS;
             if (SR > 4 && !__any(shortRow && len > 4))
-              lane_rows<(SR > 4 ? 4 : SR), false>(a, l, it, row, nullSlot, Fo, Fn, shortRow, ci,
-                                                  len, hasOut, profE, profC, profA);
+              lane_rows<(SR > 4 ? 4 : SR), false, CYC>(a, l, it, row, nullSlot, Fo, Fn, shortRow,
+                                                       ci, len, hasOut, watch, diff, miss, profE,
+                                                       profC, profA);
             else
-              lane_rows<SR, false>(a, l, it, row, nullSlot, Fo, Fn, shortRow, ci, len, hasOut,
-                                   profE, profC, profA);
+              lane_rows<SR, false, CYC>(a, l, it, row, nullSlot, Fo, Fn, shortRow, ci, len,
+                                        hasOut, watch, diff, miss, profE, profC, profA);
           }
           if (SR < kLaneRowMax && __any(midRow)) {  // wave-uniform
             const int2 *row = recL + (midRow ? rsL[ci] : 0);
-            lane_rows<kLaneRowMax, true>(a, l, it, row, nullSlot, Fo, Fn, midRow, ci,
-                                         midRow ? len : 0, hasOut, profE, profC, profA);
+            lane_rows<kLaneRowMax, true, CYC>(a, l, it, row, nullSlot, Fo, Fn, midRow, ci,
+                                              midRow ? len : 0, hasOut, watch, diff, miss, profE,
+                                              profC, profA);
           }
         }
         /* longer rows: one wave per frontier vertex */
@@ -1686,6 +1746,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
             if (lane == 0) {
               const float oldLabel = Fo[ci];
               const float nl = dlp::new_label(W, S, oldLabel);
+              if (CYC) diff = diff || !same_bits(nl, Fn[ci]);
               Fn[ci] = nl;
               changed = fabsf(nl - oldLabel) > a.delta;
               profE += (unsigned)len;
@@ -1700,7 +1761,9 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
               else if (p == len) t = ci;  // the vertex itself
               bool appL = false;
               if (t < nCore) {
-                appL = atomicMax(&stampL[t], it.stampNextL) < it.stampNextL;
+                const int old = atomicMax(&it.stampL[t], it.stampNextL);
+                appL = old < it.stampNextL;
+                if (CYC) miss = miss || (appL && old != it.stampNextL - 2);
               } else if (t < nCore + nHE) {
                 profA += mark_outside(a, l, it, haloE[t - nCore]);
               }
@@ -1709,6 +1772,10 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
               if (slot >= 0) it.qout[slot] = t;
             }
           }
+        }
+        if (CYC) {
+          if (__any(diff) && lane == 0) sh[SH_LASTDIFF] = k;
+          if (__any(miss) && lane == 0) sh[SH_LASTMISS] = k;
         }
         __syncthreads();
         ++k;
@@ -1725,7 +1792,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
         g = gidL[i];
         a.lab0[g] = lab0L[i];
         a.lab1[g] = lab1L[i];
-        const int st = stampL[i];
+        const int st = max(stampL[i], stampOdd[i]);
         if (st != DLP_INT_MAX && st > kBuild) {  // entered a frontier here
           const int old = atomicMax(&a.iterStamp[g], stampBase + k);
           first = old < stampBase;
@@ -1802,8 +1869,8 @@ __global__ __launch_bounds__(LT) void k_propagate_local(PropArgs a, LocalArgs l,
   if (threadIdx.x < 64) S.dummyStamp[threadIdx.x] = DLP_INT_MAX;  // first pass starts with a barrier
   LocalProf prof;
   int k = k0;
-  const int reason = local_passes<LT, SR, OWNER, MASK>(a, l, k, maxIter, (int *)pool4, S, prof,
-                                                 OWNER ? -1 : l.ownerAfter);
+  const int reason = local_passes<LT, SR, OWNER, MASK, false>(
+      a, l, k, maxIter, maxIter, (int *)pool4, S, prof, OWNER ? -1 : l.ownerAfter);
   if (threadIdx.x == 0) {
     a.ctr->nextIter = k;
     a.ctr->localReason = reason;
@@ -2081,7 +2148,9 @@ __global__ __launch_bounds__(LT) void k_propagate_multi(const GraphProp *graphs)
         exitCode = k;
         break;
       }
-      const int reason = local_passes<LT, SR, false>(a, l, k, stopAt, (int *)pool4, S, lprof, -1);
+      const int reason =
+          local_passes<LT, SR, false, false, true>(a, l, k, stopAt, maxIter, (int *)pool4, S,
+                                                   lprof, -1);
       if (reason == DLP_LOCAL_CAPPED) more = true;
       if (reason != DLP_LOCAL_TOO_BIG) break;
       resumeAt = k + backoff;

@@ -125,3 +125,28 @@ def test_trace_runs_every_iteration(gpu_available):
             orc.run_batch(b)
             assert np.array_equal(tr.snapshot()["frontierSizes"], orc.frontier_sizes())
         assert ctx.skipped() == (0, 0)
+
+
+@pytest.mark.parametrize("cap", CAPS)
+@pytest.mark.parametrize("slices", [0, 700])
+@pytest.mark.parametrize("shape", [3, 1, 5])
+def test_shared_launch(gpu_available, tmp_path, shape, slices, cap):
+    """Many graphs in one launch (queue iterations in LDS), in lockstep and
+    stopped and resumed every 700 iterations by the serving loop."""
+    kinds = ["random", "sparse", "long rows", "one-sided"]
+    graphs = [graph(k, tmp_path) for k in kinds]
+    want = [oracle_run(k, g, cap) for k, g in zip(kinds, graphs)]
+    with L.Multi(graphs, [L.make_config(g, maxIterations=cap) for g in graphs]) as m:
+        m.set_tuning(localShape=shape)
+        if slices:
+            m.reset()
+            reqs = [(i, 0.0) for i, g in enumerate(graphs) for _ in range(g.numBatches)]
+            m.serve(reqs, sliceIterations=slices, sliceMs=-1.0, handBackAfter=-1)
+        else:
+            m.run_all()
+        m.synchronize()
+        for i, g in enumerate(graphs):
+            assert [(s["iterations"], s["updates"])
+                    for s in (m.stats(i, b) for b in range(g.numBatches))] == \
+                [r[1:] for r in want[i]], kinds[i]
+            assert np.array_equal(bits(m.labels(i)), want[i][-1][0]), kinds[i]
