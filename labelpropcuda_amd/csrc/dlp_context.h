@@ -36,6 +36,7 @@ struct dlp_context {
   float *dGtLab = nullptr, *dEW = nullptr;
   int *iterSizes = nullptr;
   int iterSizesCap = 0;
+  int *denseCount = nullptr; /* PropArgs::denseCount */
   DevCounters *pinCtr = nullptr;
   /* propBlocks 0 = by graph size; chunks of up to 1024 multi-block
    * launches (C2: 8 -> 471.9, 64 -> 498.9, 256 -> 523.5, 1024 -> 539.8 M

@@ -51,12 +51,23 @@ struct DevCounters {
   unsigned long long correct;  /* accuracy numerator                          */
   unsigned long long total;    /* accuracy denominator                        */
   int scanTotal;       /* scratch total of the last scan                      */
-  int pad[3];
+  /* flagged-frontier iterations: the last iteration recorded; the iteration
+   * found to be in the state of two iterations before (0 = none) */
+  int denseFolded, cycleIter;
+  int hubRows;         /* step API: 1 if a row is longer than blockRowMin    */
   /* LDS-resident propagation (single work-group) */
   int localGen;        /* generation of the last local build (never reset)   */
   int coreCount;       /* vertices in the saved core list (reset per batch)  */
   int nextIter;        /* iteration the local kernel stopped at              */
   int localReason;     /* why it stopped (DLP_LOCAL_*)                        */
+  /* cycle test of the flagged-frontier iterations: frontier k is marked by
+   * generation cycleBase + 1 + k (< 0: no test in this batch); the last
+   * iteration that changed a label bit, and the last whose frontier is not
+   * known to be made of vertices of the one two before (both at least
+   * kCycleFrom); the sizes of the last frontiers, by k & 3 */
+  int cycleBase, lastDiff, lastMiss;
+  int denseSize[4];
+  int pad;
   /* propagation work counters, accumulated while profiling is on */
   unsigned long long profEdges;        /* row entries read by frontier vertices */
   unsigned long long profChangedEdges; /* (row length + 1) of changed vertices  */

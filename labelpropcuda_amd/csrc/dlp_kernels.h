@@ -47,7 +47,24 @@ struct PropArgs {
    * for bit are counted instead of run (dlp_cycle_skip); 0 while every
    * iteration's frontier size is recorded */
   int cycles;
+  /* nullable: the flagged-frontier iterations' flags of even and odd
+   * frontiers (N bytes each, padded to whole words; the LDS kernels' coreIdx
+   * and haloIdx, whose contents mean nothing between their launches) and the
+   * counters of kDenseCountInts ints */
+  uint8_t *flag0, *flag1;
+  int *denseCount;
+  /* membership marks of even and odd frontiers for the cycle test of the
+   * flagged-frontier iterations, N each: the LDS kernels' core and halo
+   * generations, a mark being a generation number of its own, reserved when
+   * the batch starts (DevCounters::cycleBase) */
+  int *mark0, *mark1;
 };
+/* flagged-frontier iterations look for cycles from this iteration on: a
+ * batch that converges does so in a few hundred iterations and then pays
+ * nothing */
+constexpr int kCycleFrom = 1024;
+/* generations a batch reserves for its frontier marks */
+__host__ __device__ inline int dlp_cycle_gens(int maxIter) { return maxIter + 2; }
 /* The frontier update is a function of its state alone: both label buffers,
  * the frontier, and which buffer is read (the parity of the iteration).  Two
  * iterations that leave every label they write as it was, between two equal
@@ -85,6 +102,31 @@ inline int dlp_auto_prop_blocks(long long numNodes) {
   return (int)(b < kMinPropagateBlocks ? kMinPropagateBlocks : (b > 8192 ? 8192 : b));
 }
 int dlp_launch_propagate(const PropArgs &a, int k, int groupLanes, int blocks, hipStream_t s);
+
+/* ---- iterations over a flagged frontier (dlp_dense.hip) ---------------- */
+constexpr int kDenseSlots = 64;
+constexpr int kDenseStride = 16; /* ints: a cache line's distance */
+constexpr int kDenseCountInts = 4 * kDenseSlots * kDenseStride;
+constexpr int kDenseThinFlags = 16;  /* flags per lane on thin frontiers */
+constexpr int kDenseMaxBlocks = 32768;
+/* whether a frontier of n among N vertices is worth walking all N flags for */
+inline bool dlp_dense_worth(long long n, long long N) { return n * 1024 >= N; }
+/* whether it is so thick that every vertex's row place, label and stamp are
+ * loaded along with its flag */
+inline bool dlp_dense_thick(long long n, long long N) { return N <= (1 << 20) || n * 16 >= N; }
+/* the queue of iteration k (n entries) -> flags */
+int dlp_launch_dense_enter(const PropArgs &a, int k, int N, int n, hipStream_t s);
+/* one iteration */
+int dlp_launch_dense(const PropArgs &a, int k, int N, bool thick, hipStream_t s);
+/* records iteration k - 1 (or the one before the cycle that was found) in the
+ * counters (denseSize: its frontier and the one before) */
+int dlp_launch_dense_fold(const PropArgs &a, int k, hipStream_t s);
+/* after a fold: flags of iteration k -> the queue, count and stamps of
+ * iteration kOut; kOut > k: the iterations between, which repeat the states
+ * of k and k - 1, are counted */
+int dlp_launch_dense_exit(const PropArgs &a, int k, int kOut, int N, hipStream_t s);
+/* the touched list from the stamps */
+int dlp_launch_dense_touched(const PropArgs &a, int N, hipStream_t s);
 
 /* global buffers of the LDS-resident propagation kernel */
 struct LocalArgs {
@@ -226,6 +268,7 @@ struct PropTiming {
 };
 
 struct PropLoopConfig {
+  int numNodes = 0;   /* length of the per-vertex arrays                     */
   int groupLanes;     /* multi-block kernel lanes per vertex                 */
   int blocks;         /* multi-block kernel grid, at most: a chunk launches
                          enough blocks for one lane group per vertex of twice
@@ -235,6 +278,8 @@ struct PropLoopConfig {
   int localThreshold; /* frontier size at or below which the LDS kernel runs */
   int maskOwnerMax;   /* owner mode starts in a register-mask kernel on
                          frontiers of at most this many vertices (<= 0 never) */
+  bool probeHubs = false; /* whether there are rows longer than blockRowMin
+                         is in the counters (hubRows)                        */
 };
 
 /* Runs propagation iterations 0 .. until the frontier empties or maxIter,
@@ -326,7 +371,8 @@ struct DBatch {
  * localGen). */
 constexpr int kMaxIterationsLimit = 1 << 28; /* larger maxIterations are rejected */
 constexpr long long kGenLimit = (1LL << 31) - 2;
-/* working-set builds of one batch, at most: a build either runs at least one
+/* generations of one batch, at most: one per iteration for the frontier
+ * marks, and one per working-set build, which either runs at least one
  * iteration, ends the launch, or is retried once without the saved core */
 inline long long dlp_gens_per_batch(int maxIter) { return 4LL * ((long long)maxIter + 1) + 4; }
 struct CounterGuardPlan {
@@ -365,7 +411,7 @@ int dlp_components(const DState &d, const DBatch &bt, hipStream_t s);
 int dlp_clear_component_ids(const DState &d, const int *ins, int n, hipStream_t s);
 int dlp_label_init(const DState &d, const DBatch &bt, hipStream_t s);
 int dlp_labels_no_edges(const DState &d, const DBatch &bt, hipStream_t s);
-int dlp_frontier0(const DState &d, int bound, hipStream_t s);
+int dlp_frontier0(const DState &d, int bound, int maxIter, hipStream_t s);
 int dlp_batch_end(const DState &d, const DBatch &bt, hipStream_t s);
 /* active CSR -> standard CSR (trace export); rowPtr N+1 */
 int dlp_export_csr(const DState &d, int *rowPtr, int *colInd, float *values, hipStream_t s);
@@ -398,8 +444,9 @@ int dlp_k_label_init(const int *rowPtr, const int *colInd, const float *values, 
                      float *p1, int *keyA, int *valA, int *keyB, int *valB, int *keyC, int *valC,
                      int *segStart, int *segEnd, float *red0, float *red1, float *W0, float *W1,
                      int *scratch, hipStream_t s);
-int dlp_k_prop_prepare(const int *isAffected, const int *status, const int *gtClass,
-                       int numNodes, int *iterStamp, int *q0, DevCounters *ctr, hipStream_t s);
+int dlp_k_prop_prepare(const int *rowPtr, const int *isAffected, const int *status,
+                       const int *gtClass, int numNodes, int hubRowMin, int *iterStamp, int *q0,
+                       DevCounters *ctr, hipStream_t s);
 int dlp_k_prop_finish(float *labels, const int *gtClass, int numNodes, int *isAffected,
                       const int *pending, DevCounters *ctr, int pendingIndex, int capped,
                       hipStream_t s);

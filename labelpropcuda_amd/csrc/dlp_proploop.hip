@@ -9,7 +9,9 @@
  *     iterations in one launch and returns when the frontier empties, the
  *     iteration cap is reached, or the working set no longer fits;
  *   - otherwise: a chunk of multi-block launches, one per iteration, whose
- *     length doubles up to maxChunk while the frontier stays large.
+ *     length doubles up to maxChunk while the frontier stays large: over a
+ *     flagged frontier (dlp_dense.hip) unless it is thin against the graph
+ *     (dlp_dense_worth) or the graph has hub rows, else over its queue.
  */
 #include <algorithm>
 
@@ -73,10 +75,11 @@ int collect_timed(PropTiming *t) {
 
 }  // namespace
 
-int dlp_run_propagation(const PropArgs &a, const LocalArgs *l, int maxIter,
+int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
                         const PropLoopConfig &cfg, DevCounters *pin, hipStream_t s,
                         PropTiming *timing, int startK) {
   int rc;
+  PropArgs a = args;
   int k = startK;
   int chunk = 2;
   int localAfter = 0; /* no local launch before this iteration (after an overflow) */
@@ -85,10 +88,35 @@ int dlp_run_propagation(const PropArgs &a, const LocalArgs *l, int maxIter,
                           that found the core too wide moves it up) */
   const int maxChunk = std::max(1, cfg.maxChunk);
   if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
+  if (cfg.probeHubs && !pin->hubRows) a.blockRowMin = 0;  // no row for the work-group tier
+  bool dense = false;     /* the frontier of iteration k is held as flags */
+  bool denseUsed = false;
+  const int N = cfg.numNodes;
+  auto leave_dense = [&](int kOut) -> int {
+    dense = false;
+    int e;
+    if ((e = dlp_launch_dense_exit(a, k, kOut, N, s)) != DLP_OK) return e;
+    k = kOut;
+    return read_ctr(a.ctr, pin, s);
+  };
   while (k < maxIter) {
-    const int n = pin->qcount[k % 3];
-    if (n == 0) break;
-    if (l && n <= cfg.localThreshold && k >= localAfter) {
+    /* with flags, the size of frontier k is not known yet: an empty frontier
+     * k - 1 has left none behind, else take that of frontier k - 2 (a
+     * frontier that lasts alternates between two) */
+    if (dense && pin->denseSize[(k - 1) & 3] == 0) {
+      dense = false;
+      break;
+    }
+    const int n = dense ? pin->denseSize[(k - 2) & 3] : pin->qcount[k % 3];
+    if (!dense && n == 0) break;
+    const bool local = l && n <= cfg.localThreshold && k >= localAfter;
+    const bool wantDense =
+        !local && a.flag0 && a.blockRowMin == 0 && dlp_dense_worth(n, N);
+    if (dense && !wantDense) {
+      if ((rc = leave_dense(k)) != DLP_OK) return rc;
+      continue;
+    }
+    if (local) {
       /* restart the core generations before a launch could carry localGen
        * past kGenLimit (one launch builds at most dlp_gens_per_batch) */
       if ((long long)pin->localGen + dlp_gens_per_batch(maxIter) >= kGenLimit &&
@@ -143,6 +171,24 @@ int dlp_run_propagation(const PropArgs &a, const LocalArgs *l, int maxIter,
         (2LL * n * cfg.groupLanes + kPropagateThreads - 1) / kPropagateThreads;
     const int blocks = (int)std::max<long long>(
         1, std::min<long long>(cfg.blocks, std::max<long long>(want, kMinPropagateBlocks)));
+    if (wantDense) {
+      const bool thick = dlp_dense_thick(n, N);
+      if (timing && (rc = begin_timed(timing, s, false, m)) != DLP_OK) return rc;
+      if (!dense && (rc = dlp_launch_dense_enter(a, k, N, n, s)) != DLP_OK) return rc;
+      dense = denseUsed = true;
+      for (int j = 0; j < m; ++j)
+        if ((rc = dlp_launch_dense(a, k + j, N, thick, s)) != DLP_OK) return rc;
+      if ((rc = dlp_launch_dense_fold(a, k + m, s)) != DLP_OK) return rc;
+      if (timing && (rc = end_timed(timing, s)) != DLP_OK) return rc;
+      k += m;
+      if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
+      chunk *= 2;
+      if (pin->cycleIter > 0) {  // the launches from there on did nothing
+        k = pin->cycleIter;
+        if ((rc = leave_dense(k + dlp_cycle_skip(k, maxIter))) != DLP_OK) return rc;
+      }
+      continue;
+    }
     PropTiming *perLaunch = (timing && !timing->perChunk) ? timing : nullptr;
     if (timing && timing->perChunk && (rc = begin_timed(timing, s, false, m)) != DLP_OK)
       return rc;
@@ -157,5 +203,7 @@ int dlp_run_propagation(const PropArgs &a, const LocalArgs *l, int maxIter,
     if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
     chunk *= 2;
   }
+  if (dense && (rc = leave_dense(k)) != DLP_OK) return rc;  // stopped at the cap
+  if (denseUsed && a.touched && (rc = dlp_launch_dense_touched(a, N, s)) != DLP_OK) return rc;
   return collect_timed(timing);
 }

@@ -248,6 +248,7 @@ namespace {
 
 int run_propagation(dlp_context *c, const PropArgs &a, int maxIter, int startK = 0) {
   PropLoopConfig cfg;
+  cfg.numNodes = c->N;
   cfg.groupLanes = c->tuning.propGroupLanes;
   cfg.blocks = c->tuning.propBlocks > 0 ? c->tuning.propBlocks : dlp_auto_prop_blocks(c->N);
   cfg.maxChunk = c->tuning.chunkIterations;
@@ -532,6 +533,7 @@ extern "C" int dlp_context_create(dlp_context **out, const dlp_config *cfg,
   TRY(c->alloc(&d.records, B));
   c->iterSizesCap = std::max(1, std::min(cfg->maxIterations, 1 << 20));
   TRY(c->alloc(&c->iterSizes, c->iterSizesCap));
+  TRY(c->alloc(&c->denseCount, kDenseCountInts));
   /* LDS-resident propagation: LDS budget, core bookkeeping, default threshold
    * = the frontier whose rows (mean degree) fill the LDS once */
   {
@@ -886,7 +888,7 @@ int dlp_ctx_batch_pre(dlp_context *c, int b, const DBatch &bt, int *markTag) {
   } else if (bt.nIns > 0) {
     if ((rc = dlp_labels_no_edges(d, bt, s)) != DLP_OK) return rc;
   }
-  return dlp_frontier0(d, c->N, s);
+  return dlp_frontier0(d, c->N, c->cfg.maxIterations, s);
 }
 
 int dlp_ctx_run_propagation(dlp_context *c, int startK) {
@@ -924,6 +926,11 @@ PropArgs dlp_ctx_prop_args(const dlp_context *c) {
    * when the full graph is */
   a.symmetric = c->symmetric ? 1 : 0;
   a.cycles = a.iterSizes ? 0 : 1;
+  a.flag0 = reinterpret_cast<uint8_t *>(c->local.coreIdx);
+  a.flag1 = reinterpret_cast<uint8_t *>(c->local.haloIdx);
+  a.denseCount = c->denseCount;
+  a.mark0 = c->local.coreGen;
+  a.mark1 = c->local.haloGen;
   return a;
 }
 

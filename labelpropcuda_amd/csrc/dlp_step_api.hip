@@ -77,11 +77,13 @@ int ws_open(Workspace **out) {
   return DLP_OK;
 }
 
-/* counters <- zero, stampBase = 1 */
-int ws_reset_counters(Workspace &w, hipStream_t s) {
+/* counters <- zero, stampBase = 1; cycleGens > 0: that many generations
+ * reserved for the frontier marks of a propagation */
+int ws_reset_counters(Workspace &w, hipStream_t s, int cycleGens = 0) {
   DevCounters z = {};
   z.stampBase = 1;
-  z.localGen = w.localGen;
+  z.localGen = w.localGen + cycleGens;
+  z.cycleBase = cycleGens > 0 ? w.localGen : -1;
   *w.pin = z;
   DLP_HIP(hipMemcpyAsync(w.ctr, w.pin, sizeof(DevCounters), hipMemcpyHostToDevice, s));
   DLP_HIP(hipStreamSynchronize(s));
@@ -294,6 +296,7 @@ struct PropScratch {
   int *stamp, *q0, *q1;
   int *coreGen; /* 2 * numNodes: core generations, then halo generations */
   int *coreIdx, *haloIdx, *coreList, *ovf;
+  int *denseCount;
   int listCap;
   int ldsBytes;
 };
@@ -308,8 +311,8 @@ int propagate_on(const PropScratch &ps, const int *rowPtr, const int *colInd, co
   int rc;
   /* both buffers equal on entry (iterativePropagation.cu:268-270) */
   if ((rc = dlp_k_copy_float(labelsBuffer, labels, numNodes, s)) != DLP_OK) return rc;
-  if ((rc = dlp_k_prop_prepare(isAffected, vertexStatus, gtClass, numNodes, ps.stamp, ps.q0,
-                               ps.ctr, s)) != DLP_OK)
+  if ((rc = dlp_k_prop_prepare(rowPtr, isAffected, vertexStatus, gtClass, numNodes,
+                               kDefaultBlockRowMin, ps.stamp, ps.q0, ps.ctr, s)) != DLP_OK)
     return rc;
   PropArgs a{};
   a.queueCap = numNodes;
@@ -330,6 +333,11 @@ int propagate_on(const PropScratch &ps, const int *rowPtr, const int *colInd, co
   a.iterSizesCap = 0;
   a.profile = 0;
   a.cycles = 1;
+  a.flag0 = reinterpret_cast<uint8_t *>(ps.coreIdx);
+  a.flag1 = reinterpret_cast<uint8_t *>(ps.haloIdx);
+  a.denseCount = ps.denseCount;
+  a.mark0 = ps.coreGen;
+  a.mark1 = ps.coreGen + numNodes;
   a.delta = delta;
   a.waveRowMin = kDefaultWaveRowMin;
   a.blockRowMin = kDefaultBlockRowMin;
@@ -347,6 +355,8 @@ int propagate_on(const PropScratch &ps, const int *rowPtr, const int *colInd, co
   l.coreList = ps.coreList;
   l.ovf = ps.ovf;
   PropLoopConfig cfg;
+  cfg.numNodes = numNodes;
+  cfg.probeHubs = true;
   cfg.groupLanes = 8;
   cfg.blocks = dlp_auto_prop_blocks(numNodes);
   cfg.maxChunk = 1024;
@@ -411,7 +421,6 @@ extern "C" int dlp_iterative_propagation(const int *rowPtr, const int *colInd,
   std::lock_guard<std::mutex> lock(g_wsMutex);
   Workspace *w;
   if ((rc = ws_open(&w)) != DLP_OK) return rc;
-  if ((rc = ws_reset_counters(*w, s)) != DLP_OK) return rc;
   if (!w->ldsBytes && (rc = dlp_local_lds_bytes(&w->ldsBytes)) != DLP_OK) return rc;
   const int listCap = dlp_local_list_cap(w->ldsBytes / 4);
   WS_BUF(int, stamp, 1, numNodes);
@@ -422,17 +431,20 @@ extern "C" int dlp_iterative_propagation(const int *rowPtr, const int *colInd,
   WS_BUF(int, haloIdx, 23, numNodes);
   WS_BUF(int, coreList, 21, listCap);
   WS_BUF(int, ovf, 22, listCap);
-  if (coreGen != w->coreGenBuf || w->sizes[19] != w->coreGenBytes) {
-    /* new or regrown buffer: restart the generations (the counters were
-     * already uploaded with the old localGen) */
+  WS_BUF(int, denseCount, 27, kDenseCountInts);
+  if (coreGen != w->coreGenBuf || w->sizes[19] != w->coreGenBytes ||
+      (long long)w->localGen + dlp_gens_per_batch(maxIterations) >= kGenLimit) {
+    /* new or regrown buffer, or generations that this call could use up:
+     * restart them */
     DLP_HIP(hipMemsetAsync(coreGen, 0, w->sizes[19], s));
-    DLP_HIP(hipMemsetAsync(&w->ctr->localGen, 0, sizeof(int), s));
     w->coreGenBuf = coreGen;
     w->coreGenBytes = w->sizes[19];
     w->localGen = 0;
   }
+  if ((rc = ws_reset_counters(*w, s, dlp_cycle_gens(std::max(maxIterations, 0)))) != DLP_OK)
+    return rc;
   const PropScratch ps{w->ctr, w->pin, stamp, q0, q1, coreGen, coreIdx, haloIdx,
-                       coreList, ovf, listCap, w->ldsBytes};
+                       coreList, ovf, denseCount, listCap, w->ldsBytes};
   rc = propagate_on(ps, rowPtr, colInd, values, labels, labelsBuffer, vertexStatus, gtClass,
                     isAffected, numNodes, delta, maxIterations, iterationsUsed, s);
   w->localGen = w->pin->localGen;
@@ -448,7 +460,8 @@ constexpr int kNoAllocMaxNodes = 1 << 19;   /* 524,288 vertices              */
 constexpr int kNoAllocListCap = 16384;      /* LDS-kernel core / overflow lists */
 constexpr long long kNoAllocCtrInts = 64;   /* 256 bytes for the counters    */
 constexpr long long kNoAllocInts =
-    kNoAllocCtrInts + 7LL * kNoAllocMaxNodes + 2LL * kNoAllocListCap; /* 14.1 MiB */
+    kNoAllocCtrInts + 7LL * kNoAllocMaxNodes + 2LL * kNoAllocListCap +
+    kDenseCountInts; /* 14.1 MiB */
 static_assert(sizeof(DevCounters) <= 4 * kNoAllocCtrInts, "counters outgrow their slot");
 
 /* The scratch of dlp_iterative_propagation_noalloc, one copy per GPU, held
@@ -461,13 +474,15 @@ std::mutex g_noAllocMutex;
 int *g_noAllocBase[kNoAllocMaxDevices];  /* device address of `scratch` per GPU */
 int g_noAllocLds[kNoAllocMaxDevices];    /* LDS bytes of the local kernel per GPU */
 
-/* counters <- zero with stampBase 1 and localGen 0; generations <- 0 */
-__global__ void k_noalloc_clear(DevCounters *ctr, int *gens, long long n) {
+/* counters <- zero with stampBase 1 and cycleGens generations reserved from 0
+ * for the frontier marks; generations <- 0 */
+__global__ void k_noalloc_clear(DevCounters *ctr, int *gens, long long n, int cycleGens) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   for (long long v = i; v < n; v += (long long)gridDim.x * blockDim.x) gens[v] = 0;
   if (i == 0) {
     DevCounters z = {};
     z.stampBase = 1;
+    z.localGen = cycleGens;
     *ctr = z;
   }
 }
@@ -537,9 +552,10 @@ extern "C" int dlp_iterative_propagation_noalloc(const int *rowPtr, const int *c
   ps.haloIdx = ps.coreIdx + N;
   ps.coreList = ps.haloIdx + N;
   ps.ovf = ps.coreList + listCap;
+  ps.denseCount = ps.ovf + listCap;
   ps.listCap = listCap;
   ps.ldsBytes = g_noAllocLds[dev];
-  if (ps.ovf + listCap > base + kNoAllocInts) {
+  if (ps.denseCount + kDenseCountInts > base + kNoAllocInts) {
     dlp_set_error_("dlp_iterative_propagation_noalloc: scratch layout overflow");
     return DLP_ERR_INTERNAL;
   }
@@ -548,7 +564,8 @@ extern "C" int dlp_iterative_propagation_noalloc(const int *rowPtr, const int *c
   /* the array keeps the previous call's contents: counters and generations
    * start from zero on every call */
   const unsigned grid = (unsigned)std::min<long long>((2 * N + 255) / 256, 4096);
-  hipLaunchKernelGGL(k_noalloc_clear, dim3(grid), dim3(256), 0, s, ps.ctr, ps.coreGen, 2 * N);
+  hipLaunchKernelGGL(k_noalloc_clear, dim3(grid), dim3(256), 0, s, ps.ctr, ps.coreGen, 2 * N,
+                     dlp_cycle_gens(std::max(maxIterations, 0)));
   DLP_LAUNCHED("k_noalloc_clear");
   return propagate_on(ps, rowPtr, colInd, values, labels, labelsBuffer, vertexStatus, gtClass,
                       isAffected, numNodes, delta, maxIterations, iterationsUsed, s);

@@ -156,7 +156,10 @@ __global__ void k_restart_gens(int *coreGen, int *haloGen, long long n, DevCount
     coreGen[v] = 0;
     haloGen[v] = 0;
   }
-  if (i == 0) ctr->localGen = 0;
+  if (i == 0) {
+    ctr->localGen = 0;
+    ctr->cycleBase = -1;  // the batch's reserved generations are gone
+  }
 }
 
 /* zero per-batch counters; clear the previous batch's per-batch flags */
@@ -177,6 +180,7 @@ __global__ void k_clear_prev(DState d, DBatch bt) {
     c->total = 0;
     c->coreCount = 0;
     c->rowCount = 0;
+    c->cycleIter = 0;
   }
   const int n1 = bt.nPrevIns, n2 = n1 + bt.nPrevDel, n3 = n2 + bt.nPrevGt;
   if (i >= n3) return;
@@ -747,8 +751,12 @@ __global__ void k_labels_no_edges(DState d, DBatch bt) {
 /* ------------------------------------------------------------------------ */
 /* frontier seeding, batch end                                              */
 /* ------------------------------------------------------------------------ */
-__global__ __launch_bounds__(kT) void k_frontier0(DState d) {
+__global__ __launch_bounds__(kT) void k_frontier0(DState d, int maxIter) {
   DevCounters *c = d.ctr;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // generations of the frontier marks
+    c->cycleBase = c->localGen;
+    c->localGen += dlp_cycle_gens(maxIter);
+  }
   const int n = c->numCand;
   const int base = c->stampBase;
   const long long gwave = ((long long)blockIdx.x * kT + threadIdx.x) >> 6;
@@ -932,21 +940,25 @@ __global__ __launch_bounds__(kT) void k_md_clean(const int *rowPtr, int *colInd,
   }
 }
 
-/* step API propagation set-up: stamps carry eligibility, first frontier */
-__global__ __launch_bounds__(kT) void k_prop_prepare(const int *isAffected, const int *status,
-                                                     const int *gtClass, int numNodes,
+/* step API propagation set-up: stamps carry eligibility, first frontier,
+ * whether a row is longer than hubRowMin */
+__global__ __launch_bounds__(kT) void k_prop_prepare(const int *rowPtr, const int *isAffected,
+                                                     const int *status, const int *gtClass,
+                                                     int numNodes, int hubRowMin,
                                                      int *iterStamp, int *q0, DevCounters *c) {
   const long long gwave = ((long long)blockIdx.x * kT + threadIdx.x) >> 6;
   const long long nwaves = ((long long)gridDim.x * kT) >> 6;
   const int lane = threadIdx.x & 63;
   for (long long v0 = gwave * 64; v0 < numNodes; v0 += nwaves * 64) {
     const long long v = v0 + lane;
-    bool in = false;
+    bool in = false, hub = false;
     if (v < numNodes) {
+      hub = rowPtr[v + 1] - rowPtr[v] > hubRowMin;
       const bool elig = status[v] == DLP_VERTEX_ACTIVE && gtClass[v] < 0;
       in = elig && isAffected[v] == 1;
       iterStamp[v] = elig ? (in ? 1 : 0) : DLP_INT_MAX;
     }
+    if (__any(hub) && lane == 0) c->hubRows = 1;
     int slot = dlp_wave_append(&c->qcount[0], in);
     if (slot >= 0) q0[slot] = (int)v;
   }
@@ -1134,8 +1146,8 @@ int dlp_labels_no_edges(const DState &d, const DBatch &bt, hipStream_t s) {
   return DLP_OK;
 }
 
-int dlp_frontier0(const DState &d, int bound, hipStream_t s) {
-  hipLaunchKernelGGL(k_frontier0, dim3(dlp_blocks(bound, kT, 2048)), dim3(kT), 0, s, d);
+int dlp_frontier0(const DState &d, int bound, int maxIter, hipStream_t s) {
+  hipLaunchKernelGGL(k_frontier0, dim3(dlp_blocks(bound, kT, 2048)), dim3(kT), 0, s, d, maxIter);
   DLP_LAUNCHED("k_frontier0");
   return DLP_OK;
 }
@@ -1291,10 +1303,11 @@ int dlp_k_label_init(const int *rowPtr, const int *colInd, const float *values, 
   return DLP_OK;
 }
 
-int dlp_k_prop_prepare(const int *isAffected, const int *status, const int *gtClass,
-                       int numNodes, int *iterStamp, int *q0, DevCounters *ctr, hipStream_t s) {
+int dlp_k_prop_prepare(const int *rowPtr, const int *isAffected, const int *status,
+                       const int *gtClass, int numNodes, int hubRowMin, int *iterStamp, int *q0,
+                       DevCounters *ctr, hipStream_t s) {
   hipLaunchKernelGGL(k_prop_prepare, dim3(dlp_blocks(numNodes, kT, 4096)), dim3(kT), 0, s,
-                     isAffected, status, gtClass, numNodes, iterStamp, q0, ctr);
+                     rowPtr, isAffected, status, gtClass, numNodes, hubRowMin, iterStamp, q0, ctr);
   DLP_LAUNCHED("k_prop_prepare");
   return DLP_OK;
 }

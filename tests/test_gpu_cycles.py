@@ -76,6 +76,8 @@ def graph(kind, tmp_path):
         return L.generate(2000, 3, 8, 3)
     if kind == "long rows":
         return star_tree(str(tmp_path / "star_"))
+    if kind == "hubs":
+        return star_tree(str(tmp_path / "hubs_"), 12, 90, 5, 8)
     return one_sided(L.generate(2000, 3, 8, 3), str(tmp_path / "one_"))
 
 
@@ -110,6 +112,50 @@ CAPS = [20000, 20001]
 ])
 def test_owner_kernels(gpu_available, tmp_path, kind, tuning, cap):
     check(kind, graph(kind, tmp_path), cap, **tuning)
+
+
+@pytest.mark.parametrize("cap", CAPS)
+@pytest.mark.parametrize("kind,tuning,skips", [
+    ("random", dict(), True),
+    ("random", dict(chunk=3), True),              # a cycle in the middle of a chunk
+    ("random", dict(chunk=1), True),
+    ("sparse", dict(), True),
+    ("one-sided", dict(), True),
+    ("long rows", dict(), True),                  # more than two entries a lane
+    ("hubs", dict(), True),                       # rows summed by a wave
+    ("hubs", dict(blockRowMin=64), False),        # hub rows: the queue kernel
+])
+def test_multi_block_kernels(gpu_available, tmp_path, kind, tuning, skips, cap):
+    """One launch per iteration, frontier as flags (or, with rows for the
+    work-group tier, as a queue, which runs every iteration)."""
+    check(kind, graph(kind, tmp_path), cap, skips, localThreshold=-1, **tuning)
+
+
+@pytest.mark.parametrize("cap", CAPS)
+def test_step_propagation(gpu_available, lib, cap):
+    """The step entry points: labels, second buffer, exit flags, iterations."""
+    import ctypes as C
+
+    import oracle.oracle as O
+    from labelpropcuda_amd import _lib
+    inp = graph("random", None)
+    o = Oracle(inp, maxIterations=cap)
+    o.run_batch(0)
+    o.run_batch(1)  # runs into the cap
+    rp, ci, vv = o.csr()
+    d, _, g = o.status()
+    init, aff = o.init_labels(), o.affected()
+    want = O.propagate(rp, ci, vv, init, d, g, aff, 1e-4, cap)
+    assert want[3] == cap
+    for fn in (lib.dlp_iterative_propagation, lib.dlp_iterative_propagation_noalloc) * 2:
+        dev = [_lib.DeviceArray(x) for x in (rp, ci, vv, init, np.zeros_like(init), d, g, aff)]
+        it = C.c_int()
+        _lib.check(fn(*[x.ptr for x in dev], inp.numNodes, C.c_float(1e-4), cap, C.byref(it),
+                      None))
+        assert it.value == cap
+        assert np.array_equal(bits(dev[3].numpy()), bits(want[0]))
+        assert np.array_equal(bits(dev[4].numpy()), bits(want[1]))
+        assert np.array_equal(dev[7].numpy(), want[2])
 
 
 def test_trace_runs_every_iteration(gpu_available):

@@ -1,0 +1,56 @@
+"""Iterations over a flagged frontier (one byte per vertex, no claims) against
+the oracle and against the queue iterations: sizes around the tiles of 64 and
+1,024 vertices, thick and thin frontiers, the touched list made from the
+stamps, the work counters and the recorded frontier sizes."""
+import numpy as np
+import pytest
+
+import labelpropcuda_amd as L
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.int32)
+
+
+@pytest.mark.parametrize("n,degree", [(63, 3), (64, 5), (65, 5), (257, 17), (1023, 4), (4099, 30)])
+@pytest.mark.parametrize("cap", [3, 400])
+def test_sizes_around_the_tiles(gpu_available, n, degree, cap):
+    inp = L.generate(n, degree, 4, n)
+    orc = Oracle(inp, maxIterations=cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        ctx.set_tuning(localThreshold=-1)  # every iteration a launch
+        tr = ctx.enable_trace(maxFrontierSizes=cap)
+        ctx.reset()
+        for b in range(inp.numBatches):
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            assert np.array_equal(tr.snapshot()["frontierSizes"], orc.frontier_sizes()), f"batch {b}"
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
+            st, ost = ctx.stats(b), orc.stats()
+            assert (st["updates"], st["accuracy"]) == (ost["updates"], ost["accuracy"])
+
+
+def test_thick_and_thin_frontiers_match_the_queue(gpu_available):
+    """1,200,003 vertices: batch 1 walks the flags in tiles of 1,024, the
+    later ones load every vertex's row place along; a wave-tier limit below
+    every hub keeps the same stream in queue iterations."""
+    inp = L.generate(1200003, 5, 6, 9)
+    runs = []
+    for blockRowMin in (-1, 64):  # flags; queue (the graph counts as having hub rows)
+        with L.Context(inp, L.make_config(inp, maxIterations=60)) as ctx:
+            ctx.set_tuning(localThreshold=-1, blockRowMin=blockRowMin)
+            ctx.set_profiling(True)
+            ctx.run_all()
+            p = ctx.prop_profile()
+            st = [ctx.stats(b) for b in range(inp.numBatches)]
+            runs.append((bits(ctx.labels()),
+                         [[s[k] for k in ("iterations", "updates", "frontier0", "numTouched",
+                                          "accuracy")] for s in st],
+                         p["edges"], p["changedEdges"]))
+    sizes = [s[1] / max(s[0], 1) for s in runs[0][1]]
+    assert min(sizes[1:]) * 16 < inp.numNodes < max(sizes) * 16
+    assert np.array_equal(runs[0][0], runs[1][0])
+    assert runs[0][1:] == runs[1][1:]
