@@ -101,6 +101,8 @@ enum {
   DLP_LOCAL_TOO_BIG = 3,   /* working set does not fit; continue multi-block */
   DLP_LOCAL_LONG = 4,      /* queue kernel ran LocalArgs::ownerAfter iterations:
                               continue with the owner kernel                 */
+  DLP_LOCAL_MOVING = 6,    /* the frontier leaves one working set after another
+                              within a few iterations; continue multi-block  */
   DLP_LOCAL_WIDE = 5       /* single-wave owner kernel: the core is too large
                               (or has long rows or ineligible vertices) for
                               it; continue with the work-group owner kernel  */

@@ -144,6 +144,9 @@ struct LocalArgs {
   int ovfCap;            /* >= ldsWords / 4                                    */
   int ldsWords;          /* dynamic LDS of the launch, in 4-byte words          */
   int shape;             /* work-group shape, [0, dlp_local_shape_count())      */
+  int minPass;           /* a launch ends (DLP_LOCAL_MOVING) when kMovingPasses
+                            passes in a row ran fewer iterations on average;
+                            0: never                                           */
   int ownerAfter;        /* iterations of a launch of the queue kernel before the
                             host goes on with the owner kernel; < 0: never     */
 };
@@ -155,6 +158,7 @@ constexpr int kLocalMaskShape = 100;
 constexpr int kMaskLevels = 3;
 constexpr int kMaskLevelThreads[kMaskLevels] = {64, 256, 512};
 constexpr int kMaskOwnerMax = 512;
+constexpr int kMovingPasses = 16;
 /* default LocalArgs::ownerAfter: only long-lived frontiers (C2's limit
  * cycles run 100,000 iterations in one launch) go on in owner mode */
 constexpr int kOwnerAfterDefault = 1024;
@@ -166,6 +170,19 @@ inline int dlp_local_list_cap(int ldsWords) { return ldsWords / 4 + 64; }
 inline int dlp_local_default_threshold(int ldsWords, long long meanDeg) {
   const long long t = ldsWords / (26 + 2 * meanDeg);
   return (int)(t < 1 ? 1 : t);
+}
+
+/* LocalArgs::minPass for a graph of N vertices.  A working set of 1,000
+ * vertices takes about 33 us to build and 1.5 to 2.5 us an iteration, a
+ * launch over the flagged frontier 5 to 6 us while the graph stays in the
+ * caches and 12 us at 6,000,000 vertices.  Without the rule and with it (two
+ * graphs each): 200,000 vertices 127/110 -> 105/96 ms, 500,000 154/167 ->
+ * 136/155, 1,000,000 70/73 -> 58/63, 6,000,000 225/229 -> 213/212.  On small
+ * graphs frontiers move in short bursts and staying away costs more: 5,000
+ * vertices 41/44 -> 46/45, 20,000 of degree 5 44 -> 51 (of degree 3 190/152
+ * -> 166/145), 50,000 99/114 -> 103/101; hence the lower end. */
+inline int dlp_local_min_pass(long long N) {
+  return N <= (1 << 16) ? 0 : (N <= (2 << 20) ? 4 : 2);
 }
 
 /* Runs propagation iterations from k in one work-group with the frontier's
@@ -278,6 +295,7 @@ struct PropLoopConfig {
   int localThreshold; /* frontier size at or below which the LDS kernel runs */
   int maskOwnerMax;   /* owner mode starts in a register-mask kernel on
                          frontiers of at most this many vertices (<= 0 never) */
+  int localMinPass = 0; /* LocalArgs::minPass                                 */
   bool probeHubs = false; /* whether there are rows longer than blockRowMin
                          is in the counters (hubRows)                        */
 };

@@ -1436,6 +1436,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
   unsigned &profU = prof.U, &profE = prof.E, &profC = prof.C, &profA = prof.A;
   unsigned long long passUpdates = 0; /* tid 0: frontier sizes of this pass */
   const int kLaunch = k;
+  int passes = 0, kPasses = k; /* passes since iteration kPasses */
 
   while (true) {  // one pass = build the LDS working set, iterate, write back
     /* every thread has read the previous pass's sh[] values */
@@ -1882,6 +1883,14 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
     if (sh[SH_BIG]) {
       reason = DLP_LOCAL_TOO_BIG;
       break;
+    }
+    if (++passes == kMovingPasses) {  // uniform
+      if (k - kPasses < kMovingPasses * l.minPass) {
+        reason = DLP_LOCAL_MOVING;
+        break;
+      }
+      passes = 0;
+      kPasses = k;
     }
     useCore = true;  // rebuild with the grown core at iteration k
   }

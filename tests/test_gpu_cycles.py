@@ -196,3 +196,22 @@ def test_shared_launch(gpu_available, tmp_path, shape, slices, cap):
                     for s in (m.stats(i, b) for b in range(g.numBatches))] == \
                 [r[1:] for r in want[i]], kinds[i]
             assert np.array_equal(bits(m.labels(i)), want[i][-1][0]), kinds[i]
+
+
+def test_moving_frontier_leaves_the_lds_kernels(gpu_available):
+    """A frontier that leaves one LDS working set after another goes on in
+    launches for a while and comes back: engine switches in the middle of a
+    batch, oracle results."""
+    inp, cap = L.generate(70000, 3, 5, 7), 1500
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        orc = Oracle(inp, maxIterations=cap)
+        ctx.set_profiling(True)
+        ctx.reset()
+        for b in range(inp.numBatches):
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            st, ost = ctx.stats(b), orc.stats()
+            assert (st["iterations"], st["updates"]) == (ost["iterations"], ost["updates"])
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
+        p = ctx.prop_profile()
+        assert p["localLaunches"] > 0 and p["launches"] > 256
