@@ -159,6 +159,10 @@ constexpr int kMaskLevels = 3;
 constexpr int kMaskLevelThreads[kMaskLevels] = {64, 256, 512};
 constexpr int kMaskOwnerMax = 512;
 constexpr int kMovingPasses = 16;
+/* LocalArgs::minPass in the shared launch: a build takes about as long as
+ * three of its work-group's HBM iterations (40 graphs of 2,000 to 16,000
+ * vertices, two seeds: without the rule 677 and 600 ms, 3: 552 and 496) */
+constexpr int kMultiMinPass = 3;
 /* default LocalArgs::ownerAfter: only long-lived frontiers (C2's limit
  * cycles run 100,000 iterations in one launch) go on in owner mode */
 constexpr int kOwnerAfterDefault = 1024;
