@@ -233,8 +233,11 @@ typedef struct dlp_batch_stats {
 
 /* Tuning knobs of the device path (0 = built-in default). */
 typedef struct dlp_tuning {
-  int propGroupLanes;   /* lanes per frontier vertex: 4, 8, 16, 32 or 64 */
-  int propBlocks;       /* most blocks of a propagation launch (a launch
+  int propGroupLanes;   /* lanes per frontier vertex: 4, 8, 16, 32 or 64
+                           (of the queue launches: thin frontiers on large
+                           graphs, graphs with hub rows; a launch over a
+                           flagged frontier has its own shape)           */
+  int propBlocks;       /* most blocks of a queue launch (a launch
                            sizes its grid to the frontier); 0 = by graph
                            size: N / 4096 within [512, 8192]            */
   int chunkIterations;  /* most multi-block iterations enqueued between

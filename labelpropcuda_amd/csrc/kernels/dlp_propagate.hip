@@ -21,7 +21,9 @@
  * Kernels implementing the same iteration:
  *   k_propagate        one launch per iteration, many work-groups, G lanes
  *                      per frontier vertex, queues / labels / stamps in HBM;
- *                      for large frontiers.
+ *                      for frontiers that are thin beside the graph and
+ *                      graphs with hub rows (the others: k_dense, in
+ *                      dlp_dense.hip, over a flagged frontier).
  *   k_propagate_local  one work-group that runs many iterations back to back
  *                      with the frontier's rows, their labels and the labels
  *                      of their neighbours staged in LDS; the limit cycles
