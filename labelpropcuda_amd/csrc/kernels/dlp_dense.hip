@@ -58,6 +58,18 @@ __device__ __forceinline__ float group_sum8(float x) {
   return x + lane_above<1>(x);
 }
 
+/* vertex at position `at` of a tile: beyond INT_MAX behind the last vertex of
+ * a graph of nearly 2^31, hence unsigned */
+__host__ __device__ constexpr unsigned dense_vertex(int tile, int perTile, int at) {
+  return (unsigned)tile * (unsigned)perTile + (unsigned)at;
+}
+/* flag words of N vertices */
+__host__ __device__ constexpr int dense_words(int N) { return (int)(((unsigned)N + 3u) / 4u); }
+static_assert(dense_vertex(DLP_INT_MAX / 1024, 1024, 1023) >= (unsigned)DLP_INT_MAX &&
+                  dense_vertex(DLP_INT_MAX / 64, 64, 63) >= (unsigned)DLP_INT_MAX &&
+                  dense_words(DLP_INT_MAX) == 1 << 29,
+              "the last tile of the largest graph");
+
 struct DenseProf {
   unsigned E = 0, C = 0, A = 0;
 };
@@ -227,14 +239,14 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
   for (int tile = gwave; tile < tiles; tile += nwaves) {  // wave-uniform
     const int base = tile * (64 * VPL);
     if constexpr (VPL == 1) {
-      const int v = base + lane;
-      const bool in = v < N;
+      const unsigned v = dense_vertex(tile, 64, lane);
+      const bool in = v < (unsigned)N;
       const int f = in ? cur[v] : 0;
       const int stamp = in ? a.iterStamp[v] : DLP_INT_MAX;
       const float old = in ? Fold[v] : 0.0f;
       const float now = (WATCH && in) ? Fnew[v] : 0.0f;
       int beg = 0, len = 0;
-      if (in) dense_row(a, v, beg, len);
+      if (in) dense_row(a, (int)v, beg, len);
       if (f) cur[v] = 0;
       const bool act = f && stamp != DLP_INT_MAX;
       const unsigned long long m = dlp_ballot(act);
@@ -262,10 +274,10 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
       constexpr int WPL = VPL / 4;
       unsigned w[WPL];
       int c = 0;
-      const int v0 = base + lane * VPL;
+      const unsigned v0 = dense_vertex(tile, 64 * VPL, lane * VPL);
 #pragma unroll
       for (int j = 0; j < WPL; ++j) {  // the arrays are padded to whole words
-        w[j] = v0 + 4 * j < N ? reinterpret_cast<const unsigned *>(cur)[(v0 >> 2) + j] : 0u;
+        w[j] = v0 + 4 * j < (unsigned)N ? reinterpret_cast<const unsigned *>(cur)[(v0 >> 2) + j] : 0u;
         c += __popc(w[j]);  // a flag byte is 0 or 1
       }
       const int incl = dlp_wave_inclusive_sum(c);
@@ -338,7 +350,7 @@ __global__ __launch_bounds__(64) void k_dense_fold(PropArgs a, int k) {
 /* flags and counts to zero before iteration k */
 __global__ __launch_bounds__(kDT) void k_dense_clear(PropArgs a, int k, int N) {
   const int i = (int)(blockIdx.x * kDT + threadIdx.x), stride = (int)(gridDim.x * kDT);
-  for (int w = i; w < (N + 3) / 4; w += stride) {
+  for (int w = i; w < dense_words(N); w += stride) {
     reinterpret_cast<unsigned *>(a.flag0)[w] = 0u;
     reinterpret_cast<unsigned *>(a.flag1)[w] = 0u;
   }
@@ -367,7 +379,8 @@ __global__ __launch_bounds__(kDT) void k_dense_exit(PropArgs a, int k, int kOut,
     DevCounters *c = a.ctr;
     const unsigned long long sum =
         (unsigned long long)((kOut - k) / 2) *
-        (unsigned long long)(c->denseSize[(k - 2) & 3] + c->denseSize[(k - 1) & 3]);
+        ((unsigned long long)c->denseSize[(k - 2) & 3] +
+         (unsigned long long)c->denseSize[(k - 1) & 3]);
     if (kOut > k) c->iterUsed = kOut;
     c->updates += sum;
     c->skippedIterations += (unsigned long long)(kOut - k);
@@ -378,7 +391,7 @@ __global__ __launch_bounds__(kDT) void k_dense_exit(PropArgs a, int k, int kOut,
   const uint8_t *cur = (k & 1) ? a.flag1 : a.flag0;
   int *q = (k & 1) ? a.q1 : a.q0;
   const int stamp = a.ctr->stampBase + kOut;
-  const int words = (N + 3) / 4;
+  const int words = dense_words(N);
   const int wave0 = (int)((blockIdx.x * kDT + threadIdx.x) & ~63u);
   const int lane = threadIdx.x & 63, stride = (int)(gridDim.x * kDT);
   for (int b = wave0; b < words; b += stride) {  // wave-uniform
