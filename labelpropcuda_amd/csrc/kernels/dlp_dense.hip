@@ -58,17 +58,9 @@ __device__ __forceinline__ float group_sum8(float x) {
   return x + lane_above<1>(x);
 }
 
-/* vertex at position `at` of a tile: beyond INT_MAX behind the last vertex of
- * a graph of nearly 2^31, hence unsigned */
-__host__ __device__ constexpr unsigned dense_vertex(int tile, int perTile, int at) {
-  return (unsigned)tile * (unsigned)perTile + (unsigned)at;
-}
-/* flag words of N vertices */
+/* flag words of N vertices (N + 3 is beyond INT_MAX on the largest graphs) */
 __host__ __device__ constexpr int dense_words(int N) { return (int)(((unsigned)N + 3u) / 4u); }
-static_assert(dense_vertex(DLP_INT_MAX / 1024, 1024, 1023) >= (unsigned)DLP_INT_MAX &&
-                  dense_vertex(DLP_INT_MAX / 64, 64, 63) >= (unsigned)DLP_INT_MAX &&
-                  dense_words(DLP_INT_MAX) == 1 << 29,
-              "the last tile of the largest graph");
+static_assert(dense_words(DLP_INT_MAX) == 1 << 29, "the largest graph's flags");
 
 struct DenseProf {
   unsigned E = 0, C = 0, A = 0;
@@ -239,14 +231,14 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
   for (int tile = gwave; tile < tiles; tile += nwaves) {  // wave-uniform
     const int base = tile * (64 * VPL);
     if constexpr (VPL == 1) {
-      const unsigned v = dense_vertex(tile, 64, lane);
-      const bool in = v < (unsigned)N;
+      const int v = base + lane;
+      const bool in = v < N;
       const int f = in ? cur[v] : 0;
       const int stamp = in ? a.iterStamp[v] : DLP_INT_MAX;
       const float old = in ? Fold[v] : 0.0f;
       const float now = (WATCH && in) ? Fnew[v] : 0.0f;
       int beg = 0, len = 0;
-      if (in) dense_row(a, (int)v, beg, len);
+      if (in) dense_row(a, v, beg, len);
       if (f) cur[v] = 0;
       const bool act = f && stamp != DLP_INT_MAX;
       const unsigned long long m = dlp_ballot(act);
@@ -274,10 +266,10 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
       constexpr int WPL = VPL / 4;
       unsigned w[WPL];
       int c = 0;
-      const unsigned v0 = dense_vertex(tile, 64 * VPL, lane * VPL);
+      const int v0 = base + lane * VPL;
 #pragma unroll
       for (int j = 0; j < WPL; ++j) {  // the arrays are padded to whole words
-        w[j] = v0 + 4 * j < (unsigned)N ? reinterpret_cast<const unsigned *>(cur)[(v0 >> 2) + j] : 0u;
+        w[j] = v0 + 4 * j < N ? reinterpret_cast<const unsigned *>(cur)[(v0 >> 2) + j] : 0u;
         c += __popc(w[j]);  // a flag byte is 0 or 1
       }
       const int incl = dlp_wave_inclusive_sum(c);
