@@ -342,7 +342,7 @@ typedef struct dlp_prop_profile {
   double kernelMs;      /* sum of their event-measured durations            */
   int64_t edges;        /* row entries read by frontier vertices            */
   int64_t changedEdges; /* sum over changed vertices of (row length + 1)    */
-  int64_t appended;     /* next-frontier queue appends                      */
+  int64_t appended;     /* next-frontier queue appends (queue launches)     */
   /* LDS-resident kernel (many iterations per launch) */
   int64_t localLaunches;
   double localKernelMs;
@@ -365,6 +365,14 @@ typedef struct dlp_prop_profile {
 int dlp_context_set_profiling(dlp_context *ctx, int level);
 /* Profile accumulated since profiling was last turned on (synchronises). */
 int dlp_context_prop_profile(dlp_context *ctx, dlp_prop_profile *out);
+/* Of its multi-block figures, those of the launches over a flagged frontier
+ * (one flag byte per vertex, no queue); the rest are queue launches.  counts:
+ * launches; of these, thin ones (a vertex's flag alone is loaded) and idle
+ * ones (enqueued behind a cycle that was found, ended at once); frontier
+ * vertices processed, row entries read, sum over changed vertices of
+ * (row length + 1).  kernelMs is part of dlp_prop_profile's and includes
+ * setting the flags up. */
+int dlp_context_flag_profile(dlp_context *ctx, int64_t counts[6], double *kernelMs);
 
 /* Wrap-around guards of the two device counters that only grow (no
  * counterpart in the reference, whose loop restarts them per call).

@@ -244,6 +244,7 @@ SIGNATURES = {
     "dlp_context_set_trace": (C.c_int, [_VP, C.POINTER(Trace)]),
     "dlp_context_set_profiling": (C.c_int, [_VP, C.c_int]),
     "dlp_context_prop_profile": (C.c_int, [_VP, C.POINTER(PropProfile)]),
+    "dlp_context_flag_profile": (C.c_int, [_VP, i64p, C.POINTER(C.c_double)]),
     "dlp_inputs_generate": (
         C.c_int, [C.POINTER(_VP), C.c_int, C.c_int, C.c_int, C.c_uint, C.c_float, C.c_float]),
     "dlp_inputs_graph": (C.c_int, [_VP, C.POINTER(GraphView), C.POINTER(f32p)]),

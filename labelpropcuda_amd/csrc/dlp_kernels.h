@@ -276,13 +276,16 @@ __host__ __device__ inline int dlp_slice_exit(int k) { return -2 - k; }
 int dlp_launch_propagate_multi(const GraphProp *graphs, int numGraphs, int shape, int ldsWords,
                                hipStream_t s);
 
+enum PropKind : char { kPropQueue, kPropLocal, kPropFlagThin, kPropFlagThick };
 /* HIP-event timing of propagation launches (optional) */
 struct PropTiming {
   std::vector<hipEvent_t> ev; /* pairs, reused                          */
   int used = 0;
   int64_t launches = 0, localLaunches = 0;
   double ms = 0.0, localMs = 0.0;
-  std::vector<char> isLocal;  /* per pair: local kernel launch          */
+  int64_t flagLaunches = 0, flagThin = 0, flagIdle = 0; /* of launches  */
+  double flagMs = 0.0;                                  /* of ms        */
+  std::vector<char> kind;     /* per pair: PropKind                     */
   std::vector<int> count;     /* per pair: launches it brackets         */
   bool perChunk = false;      /* one pair per chunk of multi-block
                                  launches instead of one per launch     */

@@ -36,7 +36,7 @@ int read_ctr(DevCounters *dev, DevCounters *pin, hipStream_t s) {
   return DLP_OK;
 }
 
-int begin_timed(PropTiming *t, hipStream_t s, bool local, int launches) {
+int begin_timed(PropTiming *t, hipStream_t s, PropKind kind, int launches) {
   if (!t) return DLP_OK;
   while ((int)t->ev.size() < t->used + 2) {
     hipEvent_t e;
@@ -44,11 +44,11 @@ int begin_timed(PropTiming *t, hipStream_t s, bool local, int launches) {
     t->ev.push_back(e);
   }
   const int pair = t->used / 2;
-  if ((int)t->isLocal.size() < pair + 1) {
-    t->isLocal.resize(pair + 1);
+  if ((int)t->kind.size() < pair + 1) {
+    t->kind.resize(pair + 1);
     t->count.resize(pair + 1);
   }
-  t->isLocal[pair] = local ? 1 : 0;
+  t->kind[pair] = kind;
   t->count[pair] = launches;
   DLP_HIP(hipEventRecord(t->ev[t->used], s));
   return DLP_OK;
@@ -67,13 +67,19 @@ int collect_timed(PropTiming *t) {
   for (int i = 0; i < t->used; i += 2) {
     float ms = 0.0f;
     DLP_HIP(hipEventElapsedTime(&ms, t->ev[i], t->ev[i + 1]));
-    if (t->isLocal[i / 2]) {
+    const int n = t->count[i / 2];
+    const char kind = t->kind[i / 2];
+    if (kind == kPropLocal) {
       t->localMs += ms;
-      t->localLaunches += t->count[i / 2];
-    } else {
-      t->ms += ms;
-      t->launches += t->count[i / 2];
+      t->localLaunches += n;
+      continue;
     }
+    t->ms += ms;
+    t->launches += n;
+    if (kind == kPropQueue) continue;
+    t->flagMs += ms;
+    t->flagLaunches += n;
+    if (kind == kPropFlagThin) t->flagThin += n;
   }
   t->used = 0;
   return DLP_OK;
@@ -142,7 +148,7 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
         if (!a.symmetric && level > 0) level = kMaskLevels;
         if (level < kMaskLevels) la.shape = kLocalMaskShape + level;
       }
-      if ((rc = begin_timed(timing, s, true, 1)) != DLP_OK) return rc;
+      if ((rc = begin_timed(timing, s, kPropLocal, 1)) != DLP_OK) return rc;
       if ((rc = dlp_launch_propagate_local(a, la, k, maxIter, owner, s)) != DLP_OK) return rc;
       if ((rc = end_timed(timing, s)) != DLP_OK) return rc;
       if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
@@ -184,27 +190,29 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
         1, std::min<long long>(cfg.blocks, std::max<long long>(want, kMinPropagateBlocks)));
     if (wantDense) {
       const bool thick = dlp_dense_thick(n, N);
-      if (timing && (rc = begin_timed(timing, s, false, m)) != DLP_OK) return rc;
+      if ((rc = begin_timed(timing, s, thick ? kPropFlagThick : kPropFlagThin, m)) != DLP_OK)
+        return rc;
       if (!dense && (rc = dlp_launch_dense_enter(a, k, N, n, s)) != DLP_OK) return rc;
       dense = denseUsed = true;
       for (int j = 0; j < m; ++j)
         if ((rc = dlp_launch_dense(a, k + j, N, thick, s)) != DLP_OK) return rc;
       if ((rc = dlp_launch_dense_fold(a, k + m, s)) != DLP_OK) return rc;
-      if (timing && (rc = end_timed(timing, s)) != DLP_OK) return rc;
+      if ((rc = end_timed(timing, s)) != DLP_OK) return rc;
       k += m;
       if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
       chunk *= 2;
       if (pin->cycleIter > 0) {  // the launches from there on did nothing
+        if (timing) timing->flagIdle += k - pin->cycleIter;
         k = pin->cycleIter;
         if ((rc = leave_dense(k + dlp_cycle_skip(k, maxIter))) != DLP_OK) return rc;
       }
       continue;
     }
     PropTiming *perLaunch = (timing && !timing->perChunk) ? timing : nullptr;
-    if (timing && timing->perChunk && (rc = begin_timed(timing, s, false, m)) != DLP_OK)
+    if (timing && timing->perChunk && (rc = begin_timed(timing, s, kPropQueue, m)) != DLP_OK)
       return rc;
     for (int j = 0; j < m; ++j) {
-      if ((rc = begin_timed(perLaunch, s, false, 1)) != DLP_OK) return rc;
+      if ((rc = begin_timed(perLaunch, s, kPropQueue, 1)) != DLP_OK) return rc;
       if ((rc = dlp_launch_propagate(a, k + j, cfg.groupLanes, blocks, s)) != DLP_OK)
         return rc;
       if ((rc = end_timed(perLaunch, s)) != DLP_OK) return rc;

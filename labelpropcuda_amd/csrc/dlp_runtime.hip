@@ -962,12 +962,14 @@ extern "C" int dlp_context_set_profiling(dlp_context *c, int enable) {
   ctr.profLocalUpdates = ctr.profLocalEdges = ctr.profLocalChangedEdges = 0;
   ctr.profLocalAppended = ctr.profLocalOwnerUpdates = ctr.profLocalBuilds = 0;
   ctr.profLocalWaveUpdates = 0;
+  ctr.profFlagUpdates = ctr.profFlagEdges = ctr.profFlagChangedEdges = 0;
   DLP_HIP(hipMemcpy(c->d.ctr, &ctr, sizeof(ctr), hipMemcpyHostToDevice));
   c->profiling = enable;
   c->timing.perChunk = enable == 1;
   c->timing.used = 0;
   c->timing.launches = c->timing.localLaunches = 0;
-  c->timing.ms = c->timing.localMs = 0.0;
+  c->timing.ms = c->timing.localMs = c->timing.flagMs = 0.0;
+  c->timing.flagLaunches = c->timing.flagThin = c->timing.flagIdle = 0;
   return DLP_OK;
 }
 
@@ -993,6 +995,24 @@ extern "C" int dlp_context_prop_profile(dlp_context *c, dlp_prop_profile *out) {
   out->localOwnerUpdates = (int64_t)ctr.profLocalOwnerUpdates;
   out->localBuilds = (int64_t)ctr.profLocalBuilds;
   out->localWaveUpdates = (int64_t)ctr.profLocalWaveUpdates;
+  return DLP_OK;
+}
+
+extern "C" int dlp_context_flag_profile(dlp_context *c, int64_t counts[6], double *kernelMs) {
+  if (!c || !counts || !kernelMs) {
+    dlp_set_error_("dlp_context_flag_profile: NULL argument");
+    return DLP_ERR_INVALID;
+  }
+  DLP_HIP(hipStreamSynchronize(c->stream));
+  DevCounters ctr;
+  DLP_HIP(hipMemcpy(&ctr, c->d.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
+  counts[0] = c->timing.flagLaunches;
+  counts[1] = c->timing.flagThin;
+  counts[2] = c->timing.flagIdle;
+  counts[3] = (int64_t)ctr.profFlagUpdates;
+  counts[4] = (int64_t)ctr.profFlagEdges;
+  counts[5] = (int64_t)ctr.profFlagChangedEdges;
+  *kernelMs = c->timing.flagMs;
   return DLP_OK;
 }
 

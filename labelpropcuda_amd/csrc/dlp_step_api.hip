@@ -459,7 +459,7 @@ namespace {
 
 constexpr int kNoAllocMaxNodes = 1 << 19;   /* 524,288 vertices              */
 constexpr int kNoAllocListCap = 16384;      /* LDS-kernel core / overflow lists */
-constexpr long long kNoAllocCtrInts = 64;   /* 256 bytes for the counters    */
+constexpr long long kNoAllocCtrInts = 128;  /* 512 bytes for the counters    */
 constexpr long long kNoAllocInts =
     kNoAllocCtrInts + 7LL * kNoAllocMaxNodes + 2LL * kNoAllocListCap +
     kDenseCountInts; /* 14.1 MiB */

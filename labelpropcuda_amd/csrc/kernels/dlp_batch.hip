@@ -129,6 +129,9 @@ __global__ void k_reset(DState d) {
     z.profEdges = d.ctr->profEdges;  // work counters survive resets
     z.profChangedEdges = d.ctr->profChangedEdges;
     z.profAppended = d.ctr->profAppended;
+    z.profFlagUpdates = d.ctr->profFlagUpdates;
+    z.profFlagEdges = d.ctr->profFlagEdges;
+    z.profFlagChangedEdges = d.ctr->profFlagChangedEdges;
     z.profLocalUpdates = d.ctr->profLocalUpdates;
     z.profLocalEdges = d.ctr->profLocalEdges;
     z.profLocalChangedEdges = d.ctr->profLocalChangedEdges;

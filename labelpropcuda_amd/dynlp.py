@@ -412,6 +412,14 @@ class Context:
         check(self._lib.dlp_context_prop_profile(self._h, C.byref(p)))
         return {name: getattr(p, name) for name, _ in p._fields_}
 
+    def flag_profile(self) -> dict:
+        """The part of prop_profile's multi-block figures that launches over a
+        flagged frontier make up (the rest are queue launches)."""
+        c, ms = (C.c_int64 * 6)(), C.c_double()
+        check(self._lib.dlp_context_flag_profile(self._h, c, C.byref(ms)))
+        names = ("launches", "thinLaunches", "idleLaunches", "updates", "edges", "changedEdges")
+        return dict(zip(names, c), kernelMs=ms.value)
+
     def row_update(self, mode: int = -1) -> bool:
         """Sets the CSR update's row choice (0 by batch size, 1 every row, 2
         only the rows the batch can change on a symmetric graph; -1 keeps

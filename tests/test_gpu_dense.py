@@ -44,7 +44,12 @@ def test_thick_and_thin_frontiers_match_the_queue(gpu_available):
             ctx.set_tuning(localThreshold=-1, blockRowMin=blockRowMin)
             ctx.set_profiling(True)
             ctx.run_all()
-            p = ctx.prop_profile()
+            p, f = ctx.prop_profile(), ctx.flag_profile()
+            if blockRowMin < 0:  # both walks, and little else
+                assert 0 < f["thinLaunches"] < f["launches"] and f["idleLaunches"] == 0
+                assert 0.8 * p["edges"] < f["edges"] <= p["edges"]
+            else:
+                assert f == dict.fromkeys(f, 0) and p["appended"] > 0
             st = [ctx.stats(b) for b in range(inp.numBatches)]
             runs.append((bits(ctx.labels()),
                          [[s[k] for k in ("iterations", "updates", "frontier0", "numTouched",
