@@ -144,9 +144,9 @@ struct LocalArgs {
   int ovfCap;            /* >= ldsWords / 4                                    */
   int ldsWords;          /* dynamic LDS of the launch, in 4-byte words          */
   int shape;             /* work-group shape, [0, dlp_local_shape_count())      */
-  int minPass;           /* a launch ends (DLP_LOCAL_MOVING) when kMovingPasses
-                            passes in a row ran fewer iterations on average;
-                            0: never                                           */
+  int movingWork;        /* a launch ends (DLP_LOCAL_MOVING) when building passes
+                            with this many core vertices in all bought fewer than
+                            one iteration per kMovingCore of them; 0: never    */
   int ownerAfter;        /* iterations of a launch of the queue kernel before the
                             host goes on with the owner kernel; < 0: never     */
 };
@@ -158,11 +158,23 @@ constexpr int kLocalMaskShape = 100;
 constexpr int kMaskLevels = 3;
 constexpr int kMaskLevelThreads[kMaskLevels] = {64, 256, 512};
 constexpr int kMaskOwnerMax = 512;
-constexpr int kMovingPasses = 16;
-/* LocalArgs::minPass in the shared launch: a build takes about as long as
- * three of its work-group's HBM iterations (40 graphs of 2,000 to 16,000
- * vertices, two seeds: without the rule 677 and 600 ms, 3: 552 and 496) */
-constexpr int kMultiMinPass = 3;
+/* LocalArgs::movingWork.  A launch's first passes are short in
+ * any case: the core grows by the few vertices the frontier reaches until it
+ * holds them all, and then lasts for thousands of iterations (16 passes with
+ * fewer than 64 iterations took 2 such batches in 100 of update streams for a
+ * moving frontier, at up to twice their time: 400,000 vertices 9.0 -> 15.8 ms,
+ * 3,000,000 10.4 -> 18.8).  A frontier that moves makes the core outgrow the
+ * LDS and start again, for ever; the work spent on builds tells the two apart:
+ * 32 builds of 1,024 vertices take a millisecond, in which launches run 200
+ * iterations.  (32 passes of any size: one batch in 200 still 10 to 20 %
+ * slower; 64: none, but streams whose frontier does move 3 % slower.) */
+constexpr int kMovingWork = 32 << 10;
+constexpr int kMovingCore = 512;
+/* the same in the shared launch, against its work-group's HBM iterations (40
+ * graphs of 2,000 to 16,000 vertices, two seeds: without the rule 670 and
+ * 591 ms, this 531 and 493, kMovingWork 548 and 497; 24 update streams of
+ * 3,000 to 200,000 vertices 1,476, 1,198 and 1,258 ms) */
+constexpr int kMultiMovingWork = 16 << 10;
 /* default LocalArgs::ownerAfter: only long-lived frontiers (C2's limit
  * cycles run 100,000 iterations in one launch) go on in owner mode */
 constexpr int kOwnerAfterDefault = 1024;
@@ -176,18 +188,16 @@ inline int dlp_local_default_threshold(int ldsWords, long long meanDeg) {
   return (int)(t < 1 ? 1 : t);
 }
 
-/* LocalArgs::minPass for a graph of N vertices.  A working set of 1,000
- * vertices takes about 33 us to build and 1.5 to 2.5 us an iteration, a
- * launch over the flagged frontier 5 to 6 us while the graph stays in the
- * caches and 12 us at 6,000,000 vertices.  Without the rule and with it (two
- * graphs each): 200,000 vertices 127/110 -> 105/96 ms, 500,000 154/167 ->
- * 136/155, 1,000,000 70/73 -> 58/63, 6,000,000 225/229 -> 213/212.  On small
- * graphs frontiers move in short bursts and staying away costs more: 5,000
- * vertices 41/44 -> 46/45, 20,000 of degree 5 44 -> 51 (of degree 3 190/152
- * -> 166/145), 50,000 99/114 -> 103/101; hence the lower end. */
-inline int dlp_local_min_pass(long long N) {
-  return N <= (1 << 16) ? 0 : (N <= (2 << 20) ? 4 : 2);
-}
+/* Whether the loop of one graph of N vertices leaves the LDS kernels while
+ * its frontier moves (kMovingWork).  A working set of 1,000 vertices takes
+ * about 33 us to build and 1.5 to 2.5 us an iteration, a launch over the
+ * flagged frontier 4.5 to 6 us while the graph stays in the caches.  Without
+ * the rule and with it, whole streams: 100,000 vertices of degree 3 435 ->
+ * 378 ms, 200,000 of degree 5 204 -> 190, 1,000,000 57 -> 52, 3,000,000 126
+ * -> 109.  On smaller graphs frontiers move in short bursts (16 passes: 5,000
+ * vertices 41/44 -> 46/45 ms, 20,000 of degree 5 44 -> 51, of degree 3
+ * 190/152 -> 166/145, 50,000 99/114 -> 103/101), hence the lower end. */
+inline bool dlp_local_leaves_moving(long long N) { return N > (1 << 16); }
 
 /* Runs propagation iterations from k in one work-group with the frontier's
  * rows and neighbour labels held in LDS, until the frontier empties, k
@@ -302,7 +312,7 @@ struct PropLoopConfig {
   int localThreshold; /* frontier size at or below which the LDS kernel runs */
   int maskOwnerMax;   /* owner mode starts in a register-mask kernel on
                          frontiers of at most this many vertices (<= 0 never) */
-  int localMinPass = 0; /* LocalArgs::minPass                                 */
+  bool leaveMoving = false; /* dlp_local_leaves_moving                        */
   bool probeHubs = false; /* whether there are rows longer than blockRowMin
                          is in the counters (hubRows)                        */
 };

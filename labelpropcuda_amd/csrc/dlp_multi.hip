@@ -157,7 +157,7 @@ GraphProp graph_prop(const dlp_multi *m, int gi) {
   g.a = dlp_ctx_prop_args(c);
   g.l = c->local;
   g.l.ldsWords = m->ldsWords;
-  g.l.minPass = kMultiMinPass;
+  g.l.movingWork = kMultiMovingWork;
   g.maxIter = c->cfg.maxIterations;
   const long long th = (long long)c->tuning.localThreshold * m->thresholdPct / 100;
   g.threshold =

@@ -20,9 +20,8 @@
 namespace {
 
 /* iterations the LDS kernels are left for once the frontier was seen to move
- * through their working sets (64 ran into the same again on a 50,000-vertex
- * stream: 102.7 and 110.0 ms on two graphs against 102.9 and 101.2; doubling
- * up to 1,024 stayed away too long: 115.3 and 131.0) */
+ * through their working sets (128 doubling to 512 instead: 50,000 to
+ * 3,000,000-vertex streams the same within 1 %) */
 constexpr int kMovingAway = 256;
 
 int read_ctr(DevCounters *dev, DevCounters *pin, hipStream_t s) {
@@ -138,7 +137,7 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
        * core of about twice the frontier (a limit cycle alternates between
        * two frontiers), at least maskMin */
       LocalArgs la = *l;
-      la.minPass = cfg.localMinPass;
+      la.movingWork = cfg.leaveMoving ? kMovingWork : 0;
       int level = kMaskLevels;
       if (owner && n <= std::min(cfg.maskOwnerMax, kMaskOwnerMax)) {
         level = maskMin;
@@ -162,10 +161,7 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
         chunk = 2;
         owner = false;
       }
-      if (pin->localReason == DLP_LOCAL_MOVING) {
-        localAfter = next + kMovingAway;
-        chunk = kMovingAway;
-      }
+      if (pin->localReason == DLP_LOCAL_MOVING) localAfter = next + kMovingAway;
       if (pin->localReason == DLP_LOCAL_LONG) {
         owner = true;
         maskMin = 0;
@@ -179,7 +175,9 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
       continue;
     }
     chunk = std::min(chunk, maxChunk);
-    const int m = std::min(chunk, maxIter - k);
+    int m = std::min(chunk, maxIter - k);
+    /* not past the iteration from which the LDS kernel may run again */
+    if (l && n <= cfg.localThreshold && k < localAfter) m = std::min(m, localAfter - k);
     /* grid: one lane group per vertex of twice the chunk's first frontier
      * (frontiers grow within a chunk), at least kMinPropagateBlocks (a small
      * frontier spread over many compute units hides latency better than

@@ -249,7 +249,7 @@ namespace {
 int run_propagation(dlp_context *c, const PropArgs &a, int maxIter, int startK = 0) {
   PropLoopConfig cfg;
   cfg.numNodes = c->N;
-  cfg.localMinPass = dlp_local_min_pass(c->N);
+  cfg.leaveMoving = dlp_local_leaves_moving(c->N);
   cfg.groupLanes = c->tuning.propGroupLanes;
   cfg.blocks = c->tuning.propBlocks > 0 ? c->tuning.propBlocks : dlp_auto_prop_blocks(c->N);
   cfg.maxChunk = c->tuning.chunkIterations;

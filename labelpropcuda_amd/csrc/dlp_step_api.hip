@@ -356,7 +356,7 @@ int propagate_on(const PropScratch &ps, const int *rowPtr, const int *colInd, co
   l.ovf = ps.ovf;
   PropLoopConfig cfg;
   cfg.numNodes = numNodes;
-  cfg.localMinPass = dlp_local_min_pass(numNodes);
+  cfg.leaveMoving = dlp_local_leaves_moving(numNodes);
   cfg.probeHubs = true;
   cfg.groupLanes = 8;
   cfg.blocks = dlp_auto_prop_blocks(numNodes);

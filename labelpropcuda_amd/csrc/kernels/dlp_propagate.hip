@@ -419,6 +419,8 @@ enum {
   SH_LASTDIFF, /* queue iterations: the last one that changed a label bit,   */
   SH_LASTMISS, /* and the last one whose next frontier is not known to be
                   made of vertices of the frontier two before it             */
+  SH_BUILT,   /* core vertices built since iteration SH_KBUILT               */
+  SH_KBUILT,
   SH_COUNT
 };
 
@@ -1438,7 +1440,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
   unsigned &profU = prof.U, &profE = prof.E, &profC = prof.C, &profA = prof.A;
   unsigned long long passUpdates = 0; /* tid 0: frontier sizes of this pass */
   const int kLaunch = k;
-  int passes = 0, kPasses = k; /* passes since iteration kPasses */
+  if (tid == 0) sh[SH_BUILT] = DLP_INT_MAX;  // starts over below
 
   while (true) {  // one pass = build the LDS working set, iterate, write back
     /* every thread has read the previous pass's sh[] values */
@@ -1462,6 +1464,10 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       sh[SH_NLONG0] = 0;
       sh[SH_NLONG1] = 0;
       sh[SH_INELIG] = 0;
+      if (sh[SH_BUILT] >= l.movingWork) {
+        sh[SH_BUILT] = 0;
+        sh[SH_KBUILT] = k;
+      }
       sh[SH_LASTACT] = sh[SH_LASTDIFF] = sh[SH_LASTMISS] = k;
     }
     __syncthreads();
@@ -1868,6 +1874,7 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
         c->qcount[k % 3] = nl + no;
         c->qcount[(k + 1) % 3] = 0;
         c->coreCount = min(nCore, l.coreListCap);
+        sh[SH_BUILT] += nCore;
         if (k > kBuild) {  // iterations kBuild .. k-1 ran
           c->iterUsed = k;
           c->updates += passUpdates;
@@ -1886,13 +1893,10 @@ __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &
       reason = DLP_LOCAL_TOO_BIG;
       break;
     }
-    if (++passes == kMovingPasses) {  // uniform
-      if (k - kPasses < kMovingPasses * l.minPass) {
-        reason = DLP_LOCAL_MOVING;
-        break;
-      }
-      passes = 0;
-      kPasses = k;
+    if (l.movingWork > 0 && sh[SH_BUILT] >= l.movingWork &&
+        k - sh[SH_KBUILT] < l.movingWork / kMovingCore) {  // uniform
+      reason = DLP_LOCAL_MOVING;
+      break;
     }
     useCore = true;  // rebuild with the grown core at iteration k
   }
@@ -2168,8 +2172,8 @@ __device__ __forceinline__ void wg_prof_flush(const PropArgs &a, LocalProf &prof
 }
 
 /* work-group HBM iterations after a frontier was seen to move through the
- * LDS working sets (64 instead: 565 and 519 ms on the graphs of
- * kMultiMinPass) */
+ * LDS working sets (64 instead, after 16 passes: 565 and 519 ms against 552
+ * and 496 on the graphs of kMultiMovingWork) */
 constexpr int kMovingBackoff = 256;
 
 /* One work-group per graph runs the propagation of its graph's batch from

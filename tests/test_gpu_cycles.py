@@ -215,3 +215,25 @@ def test_moving_frontier_leaves_the_lds_kernels(gpu_available):
             assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
         p = ctx.prop_profile()
         assert p["localLaunches"] > 0 and p["launches"] > 256
+
+
+@pytest.mark.parametrize("degree,sizes,seed", [(4, (8091, 8727), 9), (4, (5968, 7766), 16),
+                                               (5, (6375, 6789), 7)])
+def test_growing_core_stays_in_the_lds_kernels(gpu_available, degree, sizes, seed):
+    """A small frontier whose core still grows is not one that moves: every
+    iteration of the last batch runs in the LDS kernels, to the iteration
+    cap, with the oracle's results."""
+    cap = 1500
+    inp = L.generate_stream(70001, degree, [0, *sizes], seed)
+    orc = Oracle(inp, maxIterations=cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        for b in range(inp.numBatches):
+            ctx.set_profiling(1)
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            st, ost = ctx.stats(b), orc.stats()
+            assert (st["iterations"], st["updates"]) == (ost["iterations"], ost["updates"])
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
+        assert max(orc.frontier_sizes()) <= ctx.tuning()["localThreshold"]
+        p = ctx.prop_profile()
+        assert st["iterations"] == cap and p["localLaunches"] > 0 and p["launches"] == 0
