@@ -111,9 +111,20 @@ constexpr int kDenseThinFlags = 16;  /* flags per lane on thin frontiers */
 constexpr int kDenseMaxBlocks = 32768;
 /* whether a frontier of n among N vertices is worth walking all N flags for */
 inline bool dlp_dense_worth(long long n, long long N) { return n * 1024 >= N; }
-/* whether it is so thick that every vertex's row place, label and stamp are
- * loaded along with its flag */
-inline bool dlp_dense_thick(long long n, long long N) { return N <= (1 << 20) || n * 16 >= N; }
+/* Whether it is so thick that every vertex's row place, label and stamp are
+ * loaded along with its flag: 20 bytes for each of N vertices, against one
+ * more round trip and lanes left idle for each flagged one.  us a launch,
+ * thick and thin, over frontiers of one vertex in so many:
+ *     500,000 vertices   in 400  4.9  4.6   in 200  5.4   5.8   in 70  6.1   7.7
+ *   1,000,000            in 200  7.0  5.7   in 70   8.9   8.1   in 53  9.9   9.8
+ *                        in 25  12.0 15.8
+ *   2,000,000            in 100 14.0  8.3   in 38  18.2  14.5   in 19 22.2  22.4
+ *   6,000,000            in 77  36.3 17.8   in 19  56.5  52.8   in 13 70.3  68.5
+ * Up to 250,000 vertices thick is never behind by more than 0.1; at 1,500,000
+ * one in 64 is too early (two streams 134 and 152 ms, against 140 and 162). */
+inline bool dlp_dense_thick(long long n, long long N) {
+  return N <= (1 << 19) || n * (N <= (1 << 20) ? 64 : 16) >= N;
+}
 /* the queue of iteration k (n entries) -> flags */
 int dlp_launch_dense_enter(const PropArgs &a, int k, int N, int n, hipStream_t s);
 /* one iteration */
@@ -160,10 +171,9 @@ constexpr int kMaskLevelThreads[kMaskLevels] = {64, 256, 512};
 constexpr int kMaskOwnerMax = 512;
 /* LocalArgs::movingWork.  A launch's first passes are short in
  * any case: the core grows by the few vertices the frontier reaches until it
- * holds them all, and then lasts for thousands of iterations (16 passes with
- * fewer than 64 iterations took 2 such batches in 100 of update streams for a
- * moving frontier, at up to twice their time: 400,000 vertices 9.0 -> 15.8 ms,
- * 3,000,000 10.4 -> 18.8).  A frontier that moves makes the core outgrow the
+ * holds them all, and then lasts for thousands of iterations (told by 16
+ * passes with fewer than 64 iterations, such batches took up to twice their
+ * time: 400,000 vertices 9.0 -> 15.8 ms, 3,000,000 10.4 -> 18.8).  A frontier that moves makes the core outgrow the
  * LDS and start again, for ever; the work spent on builds tells the two apart:
  * 32 builds of 1,024 vertices take a millisecond, in which launches run 200
  * iterations.  (32 passes of any size: one batch in 200 still 10 to 20 %

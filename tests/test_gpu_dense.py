@@ -59,3 +59,22 @@ def test_thick_and_thin_frontiers_match_the_queue(gpu_available):
     assert min(sizes[1:]) * 16 < inp.numNodes < max(sizes) * 16
     assert np.array_equal(runs[0][0], runs[1][0])
     assert runs[0][1:] == runs[1][1:]
+
+
+@pytest.mark.parametrize("n,thin", [(1 << 19, False), ((1 << 19) + 1, True)])
+def test_walk_by_graph_size(gpu_available, n, thin):
+    """Frontiers of a few thousand: beyond 524,288 vertices flags alone are
+    walked, up to there every vertex's row place along with its flag."""
+    inp = L.generate(n, 3, 6, 9)
+    runs = []
+    for blockRowMin in (-1, 64):  # flags; queue
+        with L.Context(inp, L.make_config(inp, maxIterations=60)) as ctx:
+            ctx.set_tuning(localThreshold=-1, blockRowMin=blockRowMin)
+            ctx.set_profiling(True)
+            ctx.run_all()
+            st = [ctx.stats(b) for b in range(inp.numBatches)]
+            f = ctx.flag_profile()
+            runs.append((bits(ctx.labels()), [(s["iterations"], s["updates"]) for s in st]))
+        if blockRowMin < 0:
+            assert f["launches"] > 0 and (f["thinLaunches"] > 0) == thin
+    assert np.array_equal(runs[0][0], runs[1][0]) and runs[0][1] == runs[1][1]
