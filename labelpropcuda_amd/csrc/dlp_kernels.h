@@ -109,8 +109,24 @@ constexpr int kDenseStride = 16; /* ints: a cache line's distance */
 constexpr int kDenseCountInts = 4 * kDenseSlots * kDenseStride;
 constexpr int kDenseThinFlags = 16;  /* flags per lane on thin frontiers */
 constexpr int kDenseMaxBlocks = 32768;
-/* whether a frontier of n among N vertices is worth walking all N flags for */
+/* Whether a frontier of n among N vertices is worth walking all N flags for.
+ * A thin flagged launch is never slower than a queue launch down to a single
+ * vertex of 6,000,000 (4.7 us each; 6.4 and 7.5 at one in 1,200), but the walk
+ * grows with N alone, and frontiers that thin are about to enter the LDS
+ * kernels on any graph whose flags the caches hold. */
 inline bool dlp_dense_worth(long long n, long long N) { return n * 1024 >= N; }
+/* Whether to set flags up for it after `queued` queue launches of the batch.
+ * Setting up, reading back and the touched list cost about 45 us, a flagged
+ * launch saves 1 to 2: an excursion of a few iterations above the LDS
+ * kernels' limit stays on the queue, unless the frontier is
+ * so large that one launch saves about 5 (500,000 vertices, one in 13: 15.4
+ * and 9.2 us).  Batches with such an excursion: 1,000,000 vertices of degree 3
+ * 575 -> 511 us, 700,000 672 -> 610; long ones lose 6 launches' saving. */
+constexpr int kDenseEnterAfter = 6; /* the first chunks: 2 and 4 */
+constexpr int kDenseEnterSize = 32768;
+inline bool dlp_dense_enter(long long n, int queued) {
+  return queued >= kDenseEnterAfter || n >= kDenseEnterSize;
+}
 /* Whether it is so thick that every vertex's row place, label and stamp are
  * loaded along with its flag: 20 bytes for each of N vertices, against one
  * more round trip and lanes left idle for each flagged one.  us a launch,

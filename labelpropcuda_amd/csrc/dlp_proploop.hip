@@ -11,7 +11,8 @@
  *   - otherwise: a chunk of multi-block launches, one per iteration, whose
  *     length doubles up to maxChunk while the frontier stays large: over a
  *     flagged frontier (dlp_dense.hip) unless it is thin against the graph
- *     (dlp_dense_worth) or the graph has hub rows, else over its queue.
+ *     (dlp_dense_worth), the excursion may be a short one (dlp_dense_enter) or
+ *     the graph has hub rows, else over its queue.
  */
 #include <algorithm>
 
@@ -106,6 +107,7 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
   if (cfg.probeHubs && !pin->hubRows) a.blockRowMin = 0;  // no row for the work-group tier
   bool dense = false;     /* the frontier of iteration k is held as flags */
   bool denseUsed = false;
+  int queued = 0; /* queue launches of this call, up to kDenseEnterAfter */
   const int N = cfg.numNodes;
   auto leave_dense = [&](int kOut) -> int {
     dense = false;
@@ -125,8 +127,8 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
     const int n = dense ? pin->denseSize[(k - 2) & 3] : pin->qcount[k % 3];
     if (!dense && n == 0) break;
     const bool local = l && n <= cfg.localThreshold && k >= localAfter;
-    const bool wantDense =
-        !local && a.flag0 && a.blockRowMin == 0 && dlp_dense_worth(n, N);
+    const bool wantDense = !local && a.flag0 && a.blockRowMin == 0 && dlp_dense_worth(n, N) &&
+                           (dense || dlp_dense_enter(n, queued));
     if (dense && !wantDense) {
       if ((rc = leave_dense(k)) != DLP_OK) return rc;
       continue;
@@ -219,6 +221,7 @@ int dlp_run_propagation(const PropArgs &args, const LocalArgs *l, int maxIter,
       if ((rc = end_timed(perLaunch, s)) != DLP_OK) return rc;
     }
     if (timing && timing->perChunk && (rc = end_timed(timing, s)) != DLP_OK) return rc;
+    queued = std::min(queued + m, kDenseEnterAfter);
     k += m;
     if ((rc = read_ctr(a.ctr, pin, s)) != DLP_OK) return rc;
     chunk *= 2;

@@ -78,3 +78,22 @@ def test_walk_by_graph_size(gpu_available, n, thin):
         if blockRowMin < 0:
             assert f["launches"] > 0 and (f["thinLaunches"] > 0) == thin
     assert np.array_equal(runs[0][0], runs[1][0]) and runs[0][1] == runs[1][1]
+
+
+@pytest.mark.parametrize("cap,flagged", [(6, 0), (7, 1), (60, 54)])
+def test_flags_are_set_up_for_long_excursions(gpu_available, cap, flagged):
+    """The first six launches of a batch take the queue, in chunks of one, two or doubling."""
+    inp = L.generate(5000, 5, 4, 42)
+    orc = Oracle(inp, maxIterations=cap)
+    for b in range(3):
+        orc.run_batch(b)
+    for chunk in (1, 2, 1024):
+        with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+            ctx.set_tuning(localThreshold=-1, chunk=chunk)
+            ctx.run_batch(0)
+            ctx.run_batch(1)
+            ctx.set_profiling(1)
+            ctx.run_batch(2)
+            ctx.synchronize()
+            assert (ctx.prop_profile()["launches"], ctx.flag_profile()["launches"]) == (cap, flagged)
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels()))
