@@ -491,6 +491,8 @@ int dlp_multi_read_labels(dlp_multi *m, int graph, float *labels);
 /* per-graph record of batch b; timeMs is the all-graph batch time */
 int dlp_multi_batch_stats(dlp_multi *m, int graph, int b, dlp_batch_stats *out);
 int dlp_multi_batch_time(dlp_multi *m, int b, float *ms);
+/* dlp_context_skipped of one graph. */
+int dlp_multi_skipped(dlp_multi *m, int graph, int64_t *iterations, int64_t *updates);
 int dlp_multi_device_bytes(const dlp_multi *m, int64_t *bytes);
 
 /* Scratch pool (no counterpart in the reference, which runs one graph).

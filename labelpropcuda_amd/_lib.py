@@ -263,6 +263,7 @@ SIGNATURES = {
     "dlp_multi_read_labels": (C.c_int, [_VP, C.c_int, C.POINTER(C.c_float)]),
     "dlp_multi_batch_stats": (C.c_int, [_VP, C.c_int, C.c_int, C.POINTER(BatchStats)]),
     "dlp_multi_batch_time": (C.c_int, [_VP, C.c_int, C.POINTER(C.c_float)]),
+    "dlp_multi_skipped": (C.c_int, [_VP, C.c_int, i64p, i64p]),
     "dlp_multi_device_bytes": (C.c_int, [_VP, C.POINTER(C.c_int64)]),
     "dlp_multi_run_next": (C.c_int, [_VP, C.POINTER(C.c_int), C.c_int]),
     "dlp_multi_set_scratch_pool": (C.c_int, [_VP, C.c_int64]),

@@ -83,6 +83,31 @@ __host__ __device__ inline int dlp_cycle_gens(int maxIter) { return maxIter + 2;
  * the shared launch, 40 graphs of 2,000 to 16,000 vertices (8 batches each)
  * 1,434 -> 770 ms. */
 __host__ __device__ inline int dlp_cycle_skip(int k, int maxIter) { return (maxIter - k) & ~1; }
+/* The owner-mode kernels look for cycles in the last kCycleWindow of every
+ * kCycleEvery iterations: looking costs up to a tenth of an iteration on a
+ * small frontier, a cycle goes on for thousands and needs four in a row. */
+constexpr int kCycleEvery = 64, kCycleWindow = 6;
+__host__ __device__ inline bool dlp_cycle_look(int k) {
+  return (k & (kCycleEvery - 1)) >= kCycleEvery - kCycleWindow;
+}
+/* the first two iterations of a window: what went before them is not known */
+__host__ __device__ inline bool dlp_cycle_blind(int k) {
+  return (k & (kCycleEvery - 1)) < kCycleEvery - kCycleWindow + 2;
+}
+/* The shared launch looks in passes of their own, for the last kMultiWindow of
+ * every kMultiEvery iterations: they need more registers and a second stamp
+ * array in LDS, and a quarter more time on a small frontier (512 threads, six
+ * vertices: 1.40 against 1.10 us an iteration, also where the looking path is
+ * not taken); the rebuilds are 20 to 70 us in about 1,100. */
+constexpr int kMultiEvery = 1024, kMultiWindow = 16;
+__host__ __device__ inline bool dlp_multi_look(int k) {
+  return (k & (kMultiEvery - 1)) >= kMultiEvery - kMultiWindow;
+}
+/* the iteration at which a stretch of plain or looking passes from k ends */
+__host__ __device__ inline int dlp_multi_till(int k, bool look) {
+  const int end = (k | (kMultiEvery - 1)) + 1;
+  return look || dlp_multi_look(k) ? end : end - kMultiWindow;
+}
 constexpr int kDefaultWaveRowMin = 64;
 constexpr int kDefaultBlockRowMin = 1024;
 

@@ -919,6 +919,15 @@ extern "C" int dlp_multi_batch_time(dlp_multi *m, int b, float *ms) {
   return DLP_OK;
 }
 
+extern "C" int dlp_multi_skipped(dlp_multi *m, int g, int64_t *iterations, int64_t *updates) {
+  if (!m || g < 0 || g >= m->G) {
+    dlp_set_error_("dlp_multi_skipped: bad argument");
+    return DLP_ERR_INVALID;
+  }
+  DLP_HIP(hipStreamSynchronize(m->stream));
+  return dlp_context_skipped(m->ctx[g], iterations, updates);
+}
+
 extern "C" int dlp_multi_device_bytes(const dlp_multi *m, int64_t *bytes) {
   if (!m || !bytes) {
     dlp_set_error_("dlp_multi_device_bytes: NULL argument");

@@ -761,11 +761,15 @@ __device__ __forceinline__ int owner_iterations(
     if (tid == 0) sh[SH_QC0 + (k + 1) % 3] = 0;
     const LocalIter it{stampL, nullptr, nullptr, sh, haloE, nullptr, dumOut, nCore, nHE,
                        k + 1, stampBase + k + 1, stampBase};
-    bool act = false; /* a label bit changed, or the flag of two iterations ago differs */
+    const bool look = a.cycles && dlp_cycle_look(k);  // uniform
+    /* a label bit changed, or the flag of two iterations ago differs */
+    bool act = look && dlp_cycle_blind(k);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-      act = act || (f[v] ? 1u : 0u) != (hist[v] >> 1);
-      hist[v] = ((hist[v] << 1) & 2u) | (f[v] ? 1u : 0u);
+      if (look) {
+        act = act || (f[v] ? 1u : 0u) != (hist[v] >> 1);
+        hist[v] = ((hist[v] << 1) & 2u) | (f[v] ? 1u : 0u);
+      }
       if (!__any(f[v])) continue;  // wave-uniform
       const int ci = own[v] ? tid + v * LT : 0;
       const float oldLabel = kb ? l1[v] : l0[v];
@@ -787,7 +791,7 @@ __device__ __forceinline__ int owner_iterations(
           owner_rows<kLaneRowMax, true>(a, l, it, len[v] <= SR ? rowS : recL + ro[v], nullSlot,
                                         Fo, Fn, nxt, dumOut, lanePath, ci, len[v], hasOut[v],
                                         oldLabel, nl, changed, prof);
-        act = act || (lanePath && !same_bits(nl, kb ? l0[v] : l1[v]));
+        if (look) act = act || (lanePath && !same_bits(nl, kb ? l0[v] : l1[v]));
         l0[v] = (lanePath && kb) ? nl : l0[v];
         l1[v] = (lanePath && !kb) ? nl : l1[v];
       }
@@ -813,7 +817,7 @@ __device__ __forceinline__ int owner_iterations(
         lnl = __shfl(lnl, 0, 64);
         changed = __shfl(changed, 0, 64);
         if (lane == src) {
-          act = act || !same_bits(lnl, kb ? l0[v] : l1[v]);
+          if (look) act = act || !same_bits(lnl, kb ? l0[v] : l1[v]);
           if (kb)
             l0[v] = lnl;
           else
@@ -837,14 +841,14 @@ __device__ __forceinline__ int owner_iterations(
       *(f[v] ? &cur[ci] : dumOut) = 0;
       entered[v] = entered[v] || (f[v] && k > kBuild);
     }
-    if (__any(act) && lane == 0) sh[SH_LASTACT] = k;
+    if (look && __any(act) && lane == 0) sh[SH_LASTACT] = k;
     __syncthreads();
     const int n = sh[SH_QC0 + k % 3];
     /* the last iterations k-2 .. k left no trace: the state of k is that of
      * k - 2.  A wave already in iteration k + 1 may have stored k + 1, but
      * only after it found no cycle here, from a value that every wave finds
-     * no cycle from. */
-    const bool cycle = a.cycles && sh[SH_LASTACT] < k - 2;
+     * no cycle from.  (The blind iterations store themselves.) */
+    const bool cycle = look && !dlp_cycle_blind(k) && sh[SH_LASTACT] < k - 2;
     if (n == 0) {  // uniform
       reason = DLP_LOCAL_CONVERGED;
       break;
@@ -1063,13 +1067,14 @@ __device__ __forceinline__ int wave_owner_iterations(
     const float *Fo = kb ? lab1L : lab0L;
     float *Fn = kb ? lab0L : lab1L;
     unsigned long long cm[V];
+    const bool look = a.cycles && dlp_cycle_look(k);
     bool ch[V], anyOut = false, diff = false;
 #pragma unroll
     for (int r = 0; r < V; ++r) {
       const bool f = (fm[r] >> lane) & 1ull;
       const float old = kb ? l1[r] : l0[r];
       const float nl = mask_row_label_any<L>(src[r], w[r], Wr[r], Fo, nullSlot, f, len[r], old);
-      diff = diff || (f && !same_bits(nl, kb ? l0[r] : l1[r]));
+      if (look) diff = diff || (f && !same_bits(nl, kb ? l0[r] : l1[r]));
       ch[r] = f && fabsf(nl - old) > a.delta;
       *(f ? &Fn[lane + 64 * r] : (float *)dumOut) = nl;
       l0[r] = (f && kb) ? nl : l0[r];
@@ -1092,7 +1097,7 @@ __device__ __forceinline__ int wave_owner_iterations(
           if ((outPos[r] >> p) & 1u) prof.A += mark_outside(a, l, it, haloE[src[r][p] - nCore]);
       }
     }
-    quiet = __any(diff) ? 0 : quiet + 1;  // uniform
+    quiet = (!look || __any(diff)) ? 0 : quiet + 1;  // uniform
     /* next frontier: every changed vertex and the core vertices their rows
      * name */
     unsigned long long fm0[V]; /* frontier k */
@@ -1125,7 +1130,7 @@ __device__ __forceinline__ int wave_owner_iterations(
     if (rebuild) break;
     /* no label bit changed in the last two iterations and their frontiers
      * return: the state of iteration k is that of k - 2 */
-    if (a.cycles && quiet >= 2) {  // uniform
+    if (quiet >= 2) {  // uniform
       bool same = true;
 #pragma unroll
       for (int r = 0; r < V; ++r) same = same && fm[r] == fm1[r];
@@ -1268,7 +1273,8 @@ __device__ __forceinline__ int mask_owner_iterations(
     if (fm != 0ull)  // wave-uniform: a wave with no flagged vertex only syncs
       nl = mask_row_label_any<L>(src, w, Wrow, Fo, nullSlot, f, len, old);
     const bool ch = f && fabsf(nl - old) > a.delta;
-    const bool actW = __any(f && !same_bits(nl, kb ? l0 : l1)) || fm != fm2;
+    const bool look = a.cycles && dlp_cycle_look(k);
+    const bool actW = look && (__any(f && !same_bits(nl, kb ? l0 : l1)) || fm != fm2);
     fm2 = fm1;
     fm1 = fm;
     *(f ? &Fn[tid] : (float *)dumOut) = nl;
@@ -1317,7 +1323,7 @@ __device__ __forceinline__ int mask_owner_iterations(
 #pragma unroll
     for (int q = 0; q < W; ++q) meet |= out[q] & xc[q];
     const bool rebuild = (outs & 1) != 0;
-    quiet = (outs & 2) ? 0 : quiet + 1;
+    quiet = (!look || (outs & 2)) ? 0 : quiet + 1;
     fm = dlp_ballot(ch || meet != 0ull) & ownMask;
     if (lane == 0) S.xCount[kb][wave] = (unsigned char)__popcll(fm);
     if (tid == 0) {
@@ -1329,7 +1335,7 @@ __device__ __forceinline__ int mask_owner_iterations(
     if (rebuild) break;  // uniform
     /* iterations k-3 .. k-1 left no trace: the state of k-1 is that of k-3,
      * and so is that of k the one of k-2 */
-    const int skip = (a.cycles && quiet >= 3) ? dlp_cycle_skip(k, maxIter) : 0;
+    const int skip = quiet >= 3 ? dlp_cycle_skip(k, maxIter) : 0;
     if (skip > 0) {  // uniform: frontiers nPrev, n, nPrev, n, ... up to the cap
       const unsigned long long sum =
           (unsigned long long)(skip / 2) * (unsigned long long)(nPrev + n);
@@ -2203,7 +2209,7 @@ __global__ __launch_bounds__(LT) void k_propagate_multi(const GraphProp *graphs)
   if (threadIdx.x < 64) S.dummyStamp[threadIdx.x] = DLP_INT_MAX;
   LocalProf lprof, gprof;
   const int heavy = gp.heavy;
-  int k = kFirst, resumeAt = kFirst, exitCode = -1;
+  int k = kFirst, resumeAt = kFirst, exitCode = -1, lookFrom = 0;
   bool more = false; /* frontier of iteration k non-empty at the stop */
   if (l.ldsWords > 0 && threshold > 0) {
     while (true) {
@@ -2218,9 +2224,25 @@ __global__ __launch_bounds__(LT) void k_propagate_multi(const GraphProp *graphs)
         exitCode = k;
         break;
       }
-      const int reason =
-          local_passes<LT, SR, false, false, true>(a, l, k, stopAt, maxIter, (int *)pool4, S,
-                                                   lprof, -1);
+      /* to the end of this stretch of plain or looking passes */
+      const bool look = a.cycles && dlp_multi_look(k) && k >= lookFrom;  // uniform
+      const int till = a.cycles ? min(stopAt, dlp_multi_till(k, look)) : stopAt;
+      int reason;
+      if (look)
+        reason = local_passes<LT, SR, false, false, true>(a, l, k, till, maxIter, (int *)pool4, S,
+                                                          lprof, -1);
+      else
+        reason = local_passes<LT, SR, false, false, false>(a, l, k, till, maxIter, (int *)pool4,
+                                                           S, lprof, -1);
+      if (reason == DLP_LOCAL_CAPPED && k < stopAt) {
+        wg_global_sync();
+        continue;
+      }
+      if (look && reason == DLP_LOCAL_TOO_BIG) {  // may fit without the second stamps
+        lookFrom = till;
+        wg_global_sync();
+        continue;
+      }
       if (reason == DLP_LOCAL_CAPPED) more = true;
       if (reason != DLP_LOCAL_TOO_BIG && reason != DLP_LOCAL_MOVING) break;
       resumeAt = k + (reason == DLP_LOCAL_MOVING ? kMovingBackoff : backoff);

@@ -559,6 +559,12 @@ class Multi:
         check(self._lib.dlp_multi_batch_time(self._h, b, C.byref(ms)))
         return ms.value
 
+    def skipped(self, graph: int):
+        """Context.skipped of one graph."""
+        it, up = C.c_int64(), C.c_int64()
+        check(self._lib.dlp_multi_skipped(self._h, graph, C.byref(it), C.byref(up)))
+        return it.value, up.value
+
     def device_bytes(self) -> int:
         v = C.c_int64()
         check(self._lib.dlp_multi_device_bytes(self._h, C.byref(v)))

@@ -95,6 +95,8 @@ def check(kind, inp, cap, skips=True, **tuning):
         it, up = ctx.skipped()
         if skips:
             assert 0 < it < sum(r[1] for r in want) and 0 < up < sum(r[2] for r in want)
+        elif skips is not None:
+            assert (it, up) == (0, 0)
 
 
 CAPS = [20000, 20001]
@@ -195,6 +197,28 @@ def test_shared_launch(gpu_available, tmp_path, shape, slices, cap):
             assert [(s["iterations"], s["updates"])
                     for s in (m.stats(i, b) for b in range(g.numBatches))] == \
                 [r[1:] for r in want[i]], kinds[i]
+            assert np.array_equal(bits(m.labels(i)), want[i][-1][0]), kinds[i]
+            it, up = m.skipped(i)
+            assert 0 < it < sum(r[1] for r in want[i]) and 0 < up, kinds[i]
+
+
+@pytest.mark.parametrize("cap", [1021, 1024, 1025, 1047, 2047, 2049])
+def test_caps_around_the_looking_iterations(gpu_available, tmp_path, cap):
+    """The owner kernels look for cycles in the last 6 of 64 iterations, the
+    shared launch in passes of the last 16 of 1,024."""
+    kinds = ["random", "sparse", "long rows"]
+    graphs = [graph(k, tmp_path) for k in kinds]
+    for kind, g in zip(kinds, graphs):
+        check(kind, g, cap, None, localOwnerAfter=1)
+        check(kind, g, cap, None, localOwnerAfter=1, maskOwnerMax=-1)
+    want = [oracle_run(k, g, cap) for k, g in zip(kinds, graphs)]
+    with L.Multi(graphs, [L.make_config(g, maxIterations=cap) for g in graphs]) as m:
+        m.run_all()
+        m.synchronize()
+        for i, g in enumerate(graphs):
+            got = [(s["iterations"], s["updates"])
+                   for s in (m.stats(i, b) for b in range(g.numBatches))]
+            assert got == [r[1:] for r in want[i]], kinds[i]
             assert np.array_equal(bits(m.labels(i)), want[i][-1][0]), kinds[i]
 
 
