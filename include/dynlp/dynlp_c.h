@@ -234,9 +234,10 @@ typedef struct dlp_batch_stats {
 /* Tuning knobs of the device path (0 = built-in default). */
 typedef struct dlp_tuning {
   int propGroupLanes;   /* lanes per frontier vertex: 4, 8, 16, 32 or 64
-                           (of the queue launches: thin frontiers on large
-                           graphs, graphs with hub rows; a launch over a
-                           flagged frontier has its own shape)           */
+                           (of the queue launches: the first of a batch,
+                           thin frontiers on large graphs, graphs with
+                           hub rows; a launch over a flagged frontier
+                           has its own shape)                            */
   int propBlocks;       /* most blocks of a queue launch (a launch
                            sizes its grid to the frontier); 0 = by graph
                            size: N / 4096 within [512, 8192]            */
@@ -256,12 +257,13 @@ typedef struct dlp_tuning {
                            thread per core vertex, frontier as flags;
                            for long-lived frontiers such as limit
                            cycles): 1024 by default, -1 never            */
-  int waveRowMin;       /* multi-block kernel: rows longer than this (at
+  int waveRowMin;       /* queue launches: rows longer than this (at
                            most 64, the default) are summed by a whole
                            wave instead of the vertex's lane group       */
-  int blockRowMin;      /* multi-block kernel: rows longer than this
+  int blockRowMin;      /* queue launches: rows longer than this
                            (>= 64; default 1024) are summed by a whole
-                           work-group; -1 never                          */
+                           work-group; -1 never.  On a graph with such
+                           rows no launch walks flags                    */
   int maskOwnerMax;     /* owner mode on a frontier of at most this many
                            vertices (<= 512, the default) runs in the
                            register-mask LDS kernels (one core vertex per

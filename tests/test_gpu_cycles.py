@@ -3,6 +3,8 @@ propagation kernels count the iterations that repeat the state of two
 iterations before bit for bit instead of running them.  Labels, iteration and
 update counts must stay the oracle's, which runs every one of them, for every
 engine and for an even and an odd number of iterations left."""
+import time
+
 import numpy as np
 import pytest
 
@@ -133,6 +135,66 @@ def test_multi_block_kernels(gpu_available, tmp_path, kind, tuning, skips, cap):
     check(kind, graph(kind, tmp_path), cap, skips, localThreshold=-1, **tuning)
 
 
+def swapping_stars(k, n):
+    """k paths of six vertices, ground truth of either class at their ends,
+    among n vertices; the last batch deletes the second and the fifth and hangs
+    a seventh on the third.  That one and its two neighbours, which no other
+    vertex holds now, swap labels for ever (equal weights: with no rounding)."""
+    rng = np.random.default_rng(1)
+    base = 7 * np.arange(k, dtype=np.int32)[:, None]
+    w = rng.uniform(0.1, 1.0, (k, 6)).astype(np.float32)
+    w[:, [2, 5]] = 1.0
+    # edges 0-1, 1-2, 2-3, 3-4, 4-5 and 2-6, as rows
+    rowLen = np.zeros(n, np.int64)
+    rowLen[:7 * k] = np.tile([1, 2, 3, 2, 2, 1, 1], k)
+    col = base + np.array([1, 0, 2, 1, 3, 6, 2, 4, 3, 5, 4, 2], np.int32)
+    val = w[:, [0, 0, 1, 1, 2, 5, 2, 3, 3, 4, 4, 5]]
+    truth = np.zeros(n, np.float32)
+    truth[:7 * k] = np.tile([0, 0, 0, 1, 1, 1, 0], k)
+    ends, inner, late, gone = (base + np.array(x, np.int32)
+                               for x in ([0, 5], [1, 2, 3, 4], [6], [1, 4]))
+    none = np.zeros(0, np.int32)
+
+    def batches(*lists):
+        return np.cumsum([0] + [x.size for x in lists]).astype(np.int64), \
+            np.ascontiguousarray(np.concatenate([x.ravel() for x in lists]))
+
+    insOff, ins = batches(ends, inner, late)
+    gtOff, gtIds = batches(ends, none, none)
+    delOff, dels = batches(none, none, gone)
+    path = base + np.arange(5, dtype=np.int32)
+    eOff, eSrc = batches(none, path, base + 2)
+    return L.Inputs(
+        rowPtr=np.concatenate([[0], np.cumsum(rowLen)]).astype(np.int32),
+        colInd=col.ravel(), values=val.ravel(), trueLabels=truth, insOff=insOff, ins=ins,
+        gtOff=gtOff, gtIds=gtIds, gtLab=truth[gtIds], delOff=delOff, dels=dels, eOff=eOff,
+        eSrc=eSrc, eDst=batches(none, path + 1, base + 6)[1],
+        eW=np.concatenate([w[:, :5].ravel(), w[:, 5]]))
+
+
+@pytest.mark.parametrize("cap", [3000, 3001])
+@pytest.mark.parametrize("n,thin", [((1 << 20) + 1, True), (1 << 19, False)])
+def test_flagged_cycles_by_walk(gpu_available, n, thin, cap):
+    """A cycle of some 2,600 vertices found by the walk over flags alone (beyond
+    2^20 vertices) and by the one that loads every vertex's row place."""
+    inp = swapping_stars(6000, n)
+    orc = Oracle(inp, maxIterations=cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        ctx.set_tuning(localThreshold=-1)
+        for b in range(inp.numBatches):
+            ctx.set_profiling(1)
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            st, ost = ctx.stats(b), orc.stats()
+            assert (st["iterations"], st["updates"]) == (ost["iterations"], ost["updates"])
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
+        f = ctx.flag_profile()
+        assert st["iterations"] == cap and f["idleLaunches"] > 0
+        assert f["thinLaunches"] == (f["launches"] if thin else 0)
+        it, up = ctx.skipped()
+        assert cap - 1200 < it < cap - 1000 and up == orc.frontier_sizes()[-1] * it
+
+
 @pytest.mark.parametrize("cap", CAPS)
 def test_step_propagation(gpu_available, lib, cap):
     """The step entry points: labels, second buffer, exit flags, iterations."""
@@ -158,6 +220,15 @@ def test_step_propagation(gpu_available, lib, cap):
         assert np.array_equal(bits(dev[3].numpy()), bits(want[0]))
         assert np.array_equal(bits(dev[4].numpy()), bits(want[1]))
         assert np.array_equal(dev[7].numpy(), want[2])
+        # the same state after 40,000,000 iterations more, which run one by
+        # one would take half a minute
+        t0 = time.perf_counter()
+        dev = [_lib.DeviceArray(x) for x in (rp, ci, vv, init, np.zeros_like(init), d, g, aff)]
+        _lib.check(fn(*[x.ptr for x in dev], inp.numNodes, C.c_float(1e-4), cap + 40000000,
+                      C.byref(it), None))
+        assert it.value == cap + 40000000 and time.perf_counter() - t0 < 5.0
+        assert np.array_equal(bits(dev[3].numpy()), bits(want[0]))
+        assert np.array_equal(bits(dev[4].numpy()), bits(want[1]))
 
 
 def test_trace_runs_every_iteration(gpu_available):

@@ -5,6 +5,8 @@ set, G' in build order, CC partition and ids, iteration counts, frontier
 sizes); FP32 labels are compared bit for bit, which implies the stated 1e-5
 tolerance and the same 0.5-threshold class.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 
@@ -235,16 +237,57 @@ def hub_inputs(tmp_path, hubs=((0, 700), (1, 320))):
 
 @pytest.mark.parametrize("lanes,threshold", [(4, -1), (8, -1), (16, -1), (64, -1), (8, 0)])
 def test_rows_beyond_64_and_256_entries(gpu_available, tmp_path, lanes, threshold):
-    """The multi-block kernel sums rows of more than 64 entries with the whole
+    """The multi-block kernels sum rows of more than 64 entries with the whole
     wave (and rows past 256 entries with two positions per slot) while the
-    lane groups sum the short rows: oracle labels, iterations and frontiers
-    for every group width, with and without the LDS-resident kernel."""
+    lane groups sum the short rows: oracle labels, iterations and frontiers,
+    with and without the LDS-resident kernel.  The group width is that of a
+    batch's first six launches, the others walk flags; the queue kernel alone
+    is tested below."""
     inp = hub_inputs(tmp_path)
     deg = np.diff(np.asarray(inp.rowPtr))
     assert deg[0] >= 700 and deg[1] >= 320 and np.median(deg) < 16
     run_engine_mix(inp, 3000, groupLanes=lanes, localThreshold=threshold)
     dense = L.generate(2000, 80, 4, 5)  # most rows between 65 and 121 entries
     run_engine_mix(dense, 1000, groupLanes=lanes, localThreshold=threshold)
+
+
+def padded(inp, n):
+    """`inp` among n vertices, the others without an edge and never inserted."""
+    more = n - inp.numNodes
+    return dataclasses.replace(
+        inp, _keep=[],
+        rowPtr=np.concatenate([inp.rowPtr, np.full(more, inp.rowPtr[-1], inp.rowPtr.dtype)]),
+        trueLabels=np.concatenate([inp.trueLabels, np.zeros(more, F32)]))
+
+
+_PADDED = []  # inputs, and the oracle's labels, iterations and updates after every batch
+
+
+@pytest.mark.parametrize("lanes,waveRowMin", [(4, 64), (8, 64), (16, 64), (32, 64), (64, 64),
+                                              (4, 16), (16, 4)])
+def test_queue_launches_of_every_group_width(gpu_available, tmp_path, lanes, waveRowMin):
+    """Frontiers of less than one vertex in 1,024 stay on the queue: rows of 3
+    to 700 entries summed by every lane group and by the wave, no flags."""
+    if not _PADDED:
+        inp = padded(hub_inputs(tmp_path), 3100000)
+        orc = Oracle(inp, maxIterations=400)
+        want = []
+        for b in range(inp.numBatches):
+            orc.run_batch(b)
+            st = orc.stats()
+            want.append((bits(orc.labels()).copy(), st["iterations"], st["updates"]))
+        _PADDED.extend((inp, want))
+    inp, want = _PADDED
+    with L.Context(inp, L.make_config(inp, maxIterations=400)) as ctx:
+        ctx.set_tuning(groupLanes=lanes, waveRowMin=waveRowMin, localThreshold=-1)
+        ctx.set_profiling(1)
+        for b in range(inp.numBatches):
+            ctx.run_batch(b)
+            st = ctx.stats(b)
+            assert (st["iterations"], st["updates"]) == want[b][1:], f"batch {b}"
+            assert np.array_equal(bits(ctx.labels()), want[b][0]), f"batch {b}: labels"
+        assert ctx.prop_profile()["launches"] > 400
+        assert ctx.flag_profile()["launches"] == 0
 
 
 @pytest.mark.parametrize("waveRowMin,blockRowMin,lanes", [
@@ -254,7 +297,8 @@ def test_row_tiers_lane_wave_block(gpu_available, tmp_path, waveRowMin, blockRow
     """Rows are summed by a lane group, by a whole wave (longer than
     waveRowMin) or by a whole work-group (longer than blockRowMin): hubs of
     2,500, 1,200 and 400 entries and the degree-6 rest give the oracle's
-    labels, iterations and frontiers under every split of the three tiers."""
+    labels, iterations and frontiers under every split of the three tiers
+    (without the work-group tier, -1, most launches walk flags)."""
     inp = hub_inputs(tmp_path, hubs=((0, 2500), (3, 1200), (7, 400)))
     deg = np.diff(np.asarray(inp.rowPtr))
     assert deg[0] >= 2500 and deg[3] >= 1200 and deg[7] >= 400

@@ -128,8 +128,8 @@ def test_c3_full_stream_properties(gpu_available, c3):
     arrived[c3.ins] = True
     assert np.all(lab[~arrived] == 0.5)
     assert sum(u for _, u, _, _ in counts) > 0
-    # another engine setting: 16 lanes per frontier vertex, 2,048 blocks,
-    # chunks of 64, the LDS kernel's second work-group shape
+    # another engine setting: 16 lanes per frontier vertex and 2,048 blocks in
+    # queue launches, chunks of 64, the LDS kernel's second work-group shape
     lab2, counts2 = full_run(c3, groupLanes=16, blocks=2048, chunk=64, localShape=2)
     assert counts2 == counts, "per-batch counts differ between engine settings"
     assert np.array_equal(bits(lab2), bits(lab)), "labels differ between engine settings"
