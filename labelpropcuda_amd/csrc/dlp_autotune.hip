@@ -261,8 +261,13 @@ extern "C" int dlp_context_autotune(dlp_context *c, int trialBatches, dlp_tuning
   const int nb = trialBatches <= 0 ? c->B : std::min(trialBatches, c->B);
   dlp_tuning base = c->tuning;
   std::vector<dlp_tuning> cand;
+  /* The lane group is that of the queue launches.  Where every frontier above
+   * the LDS kernels' limit is worth flags, those are the first six of a batch
+   * only: timing three widths there picks one by noise. */
+  const bool queue = base.blockRowMin > 0 ||
+                     !dlp_dense_worth(std::max(1, base.localThreshold), c->N);
   for (int lanes : {base.propGroupLanes / 2, base.propGroupLanes, base.propGroupLanes * 2}) {
-    if (lanes < 4 || lanes > 64) continue;
+    if (lanes < 4 || lanes > 64 || (!queue && lanes != base.propGroupLanes)) continue;
     for (int shape : {1, 3}) {
       dlp_tuning t = base;
       t.propGroupLanes = lanes;

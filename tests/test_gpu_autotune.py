@@ -43,6 +43,19 @@ def test_context_autotune_keeps_results_and_fills_the_table(gpu_available, c1_in
         dynlp.tuning_table_clear()
 
 
+def test_lane_groups_stay_where_no_queue_launch_lasts(gpu_available, c1_inputs):
+    """5,000 vertices without hub rows: every frontier above the LDS kernels'
+    limit is flagged, and no lane width is chosen by noise."""
+    dynlp.tuning_table_clear()
+    try:
+        for lanes in (4, 16, 64):
+            with L.Context(c1_inputs, L.make_config(c1_inputs, maxIterations=500)) as ctx:
+                ctx.set_tuning(groupLanes=lanes)
+                assert ctx.autotune(trialBatches=4)[0]["propGroupLanes"] == lanes
+    finally:
+        dynlp.tuning_table_clear()
+
+
 def test_multi_autotune_keeps_results_and_fills_the_table(gpu_available):
     graphs = [L.generate(3000 + 700 * g, (3, 5, 7)[g % 3], 4, 60 + g) for g in range(6)]
     cfgs = [L.make_config(g, maxIterations=2000) for g in graphs]
