@@ -73,15 +73,39 @@ def propagation_bytes(updates: int, edges: int, changed_edges: int, appended: in
     return 20 * updates + 12 * edges + 4 * changed_edges + 4 * appended
 
 
-def engine_rooflines(prof: dict, updates: int) -> dict:
+def flagged_bytes(vertices: int, launches: int, updates: int, edges: int,
+                  changed_edges: int) -> int:
+    """Algorithmic bytes of iterations over a flagged frontier: one flag byte
+    per vertex and launch; per frontier vertex 21 (row start 4, row length 4,
+    stamp 4, F_old[u] 4, F_new[u] 4, its flag cleared 1) + 12 per row entry;
+    per changed vertex 1 per flag of its row entries and itself."""
+    return vertices * launches + 21 * updates + 12 * edges + changed_edges
+
+
+def with_flags(prof: dict, flags: dict) -> dict:
+    """The profile's multi-block figures split by engine: "flag", and the
+    queue launches that are left.  Launches enqueued behind a found cycle
+    ended at once; they are left out of the count, not of the time."""
+    return dict(prof, flag=dict(flags, launches=flags["launches"] - flags["idleLaunches"]),
+                launches=prof["launches"] - flags["launches"],
+                kernelMs=prof["kernelMs"] - flags["kernelMs"],
+                edges=prof["edges"] - flags["edges"],
+                changedEdges=prof["changedEdges"] - flags["changedEdges"])
+
+
+def engine_rooflines(prof: dict, updates: int, vertices: int) -> dict:
     """Per propagation kernel and step: launches, event-timed kernel time,
     mean launch time and algorithmic GB/s (the bytes above over that time).
     Multi-block launches are timed per chunk of back-to-back launches, so
-    their mean includes the dispatch gaps inside a chunk."""
-    local_u = prof["localUpdates"]
+    their mean includes the dispatch gaps inside a chunk; k_dense's also
+    includes setting up and reading back the flags."""
+    local_u, f = prof["localUpdates"], prof["flag"]
     eng = {
+        "k_dense": (f["launches"], f["kernelMs"],
+                    flagged_bytes(vertices, f["launches"], f["updates"], f["edges"],
+                                  f["changedEdges"])),
         "k_propagate": (prof["launches"], prof["kernelMs"],
-                        propagation_bytes(updates - local_u, prof["edges"],
+                        propagation_bytes(updates - local_u - f["updates"], prof["edges"],
                                           prof["changedEdges"], prof["appended"])),
         "k_propagate_local": (prof["localLaunches"], prof["localKernelMs"],
                               propagation_bytes(local_u, prof["localEdges"],
@@ -129,27 +153,32 @@ def grid_sync_costs(blocks=(64, 512), rounds: int = 2000) -> list:
     return out
 
 
-def random_access_floor_us(prof: dict, updates: int, launches: float, ra: dict) -> float:
+def random_access_floor_us(u: float, edges: float, changed: float, launches: float,
+                           ra: dict, mark_rate: str) -> float:
     """Time per multi-block launch if its random accesses ran at the measured
-    rates back to back: per vertex update the row start, row length and old
-    label loads and the new-label store, per row entry the neighbour-label
-    load, per claim (a changed vertex's entries and itself) one returning
-    atomicMax."""
-    u = updates - prof["localUpdates"]
-    loads = 3.0 * u + prof["edges"]
-    t = loads / ra["load_per_s"] + u / ra["store_per_s"] + prof["changedEdges"] / ra["atomic_max_per_s"]
+    rates back to back: per vertex update (u) the row start, row length and
+    old label loads and the new-label store, per row entry the neighbour-label
+    load, per mark (a changed vertex's entries and itself) one access at
+    `mark_rate`: a returning atomicMax in the queue, a store to a flag."""
+    t = (3.0 * u + edges) / ra["load_per_s"] + u / ra["store_per_s"] + changed / ra[mark_rate]
     return 1e6 * t / max(launches, 1.0)
 
 
 def add_random_access(engines: dict, prof: dict, updates: int, array_ints: int,
                       out: dict) -> dict:
-    """Adds the multi-block kernel's random-access floor (and its ratio to
+    """Adds the multi-block kernels' random-access floors (and their ratio to
     the measured launch time) and records the measured rates in out."""
     ra = random_access_ceilings(array_ints)
     out["random_access"] = ra
-    k = engines.get("k_propagate")
-    if k:
-        floor = random_access_floor_us(prof, updates, k["launches_per_step"], ra)
+    f = prof["flag"]
+    queued = (updates - prof["localUpdates"] - f["updates"], prof["edges"], prof["changedEdges"])
+    flagged = (f["updates"], f["edges"], f["changedEdges"])
+    for name, work, rate in (("k_propagate", queued, "atomic_max_per_s"),
+                             ("k_dense", flagged, "store_per_s")):
+        k = engines.get(name)
+        if not k:
+            continue
+        floor = random_access_floor_us(*work, k["launches_per_step"], ra, rate)
         k["random_access_floor_us"] = floor
         k["random_access_frac"] = floor / k["avg_launch_us"] if k["avg_launch_us"] else None
     return engines
@@ -580,16 +609,19 @@ def stream_main(args) -> int:
         progress(f"batch {b}: {st['iterations']} iterations, {st['updates']} updates, "
                  f"{st['timeMs']:.1f} ms")
     wall = time.perf_counter() - tw
-    timed = ctx.prop_profile()
+    timed, timed_flags = ctx.prop_profile(), ctx.flag_profile()
     updates = int(sum(s["updates"] for s in stats))
     prof = None
     if not args.no_work_counters:
         ctx.set_profiling(2)
         ctx.run_all()
         ctx.synchronize()
-        prof = ctx.prop_profile()
+        prof, flags = ctx.prop_profile(), ctx.flag_profile()
         for key in ("launches", "kernelMs", "localLaunches", "localKernelMs"):
             prof[key] = timed[key]
+        for key in ("launches", "kernelMs", "idleLaunches"):
+            flags[key] = timed_flags[key]
+        prof = with_flags(prof, flags)
         progress("work counters collected")
     repeated_iterations, repeated = ctx.skipped()
     ctx.set_profiling(0)
@@ -621,14 +653,16 @@ def stream_main(args) -> int:
         "tuning": tuning,
         "batches": [{k: s[k] for k in ("iterations", "updates", "frontier0", "numSubEdges",
                                        "numComponents", "timeMs", "accuracy")} for s in stats],
-        "propagation_time_ms": {"k_propagate": timed["kernelMs"],
+        "propagation_time_ms": {"k_propagate": timed["kernelMs"] - timed_flags["kernelMs"],
+                                "k_dense": timed_flags["kernelMs"],
                                 "k_propagate_local": timed["localKernelMs"],
-                                "launches": timed["launches"],
+                                "launches": timed["launches"] - timed_flags["launches"],
+                                "flag_launches": timed_flags["launches"],
                                 "local_launches": timed["localLaunches"]},
     }
     if prof is not None:
         out["propagation_kernels"] = add_random_access(
-            engine_rooflines(prof, updates - repeated), prof, updates - repeated, N, out)
+            engine_rooflines(prof, updates - repeated, N), prof, updates - repeated, N, out)
     if args.calibrate_copy_mib > 0:
         out["copy_calibration"] = copy_calibration(args.calibrate_copy_mib)
     print(json.dumps(out))
@@ -851,25 +885,27 @@ def main() -> int:
         updates = u
     ctx.synchronize()
     wall = time.perf_counter() - t0
-    timed = ctx.prop_profile()
+    timed, timed_flags = ctx.prop_profile(), ctx.flag_profile()
 
     # the work counters (identical every step) from one more step, outside
     # the timed region
     ctx.set_profiling(2)
     ctx.run_all()
     ctx.synchronize()
-    work = ctx.prop_profile()
+    prof, flags = ctx.prop_profile(), ctx.flag_profile()
     repeated_iterations, repeated = ctx.skipped()
     ctx.set_profiling(0)
     ctx.close()
-    prof = dict(work)
     for key in ("launches", "kernelMs", "localLaunches", "localKernelMs"):
         prof[key] = timed[key] / args.steps  # per step, from the timed region
+    for key in ("launches", "kernelMs", "idleLaunches"):
+        flags[key] = timed_flags[key] / args.steps
+    prof = with_flags(prof, flags)
 
     ms_per_step = 1000.0 * wall / args.steps
     value = updates / (wall / args.steps)
     run = updates - repeated  # updates the kernels ran: what their bytes and rates count
-    engines = engine_rooflines(prof, run)
+    engines = engine_rooflines(prof, run, args.nodes)
     ra_out = {}
     engines = add_random_access(engines, prof, run, args.nodes, ra_out)
     dominant = max(engines, key=lambda k: engines[k]["kernel_ms_per_step"])

@@ -72,8 +72,8 @@ struct DevCounters {
   unsigned long long profEdges;        /* row entries read by frontier vertices */
   unsigned long long profChangedEdges; /* (row length + 1) of changed vertices  */
   unsigned long long profAppended;     /* queue appends                         */
-  unsigned long long profFlagUpdates;  /* flagged frontier: vertices updated,   */
-  unsigned long long profFlagEdges;    /* and its part of the two above         */
+  unsigned long long profFlagUpdates;  /* the same of a flagged frontier, and   */
+  unsigned long long profFlagEdges;    /* its vertices                          */
   unsigned long long profFlagChangedEdges;
   /* the same counters for iterations run by the LDS-resident kernel */
   unsigned long long profLocalUpdates;

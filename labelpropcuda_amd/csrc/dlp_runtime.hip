@@ -983,8 +983,8 @@ extern "C" int dlp_context_prop_profile(dlp_context *c, dlp_prop_profile *out) {
   DLP_HIP(hipMemcpy(&ctr, c->d.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
   out->launches = c->timing.launches;
   out->kernelMs = c->timing.ms;
-  out->edges = (int64_t)ctr.profEdges;
-  out->changedEdges = (int64_t)ctr.profChangedEdges;
+  out->edges = (int64_t)(ctr.profEdges + ctr.profFlagEdges);
+  out->changedEdges = (int64_t)(ctr.profChangedEdges + ctr.profFlagChangedEdges);
   out->appended = (int64_t)ctr.profAppended;
   out->localLaunches = c->timing.localLaunches;
   out->localKernelMs = c->timing.localMs;

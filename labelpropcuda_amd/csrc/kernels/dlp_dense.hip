@@ -323,8 +323,6 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
       prof.A += __shfl_xor(prof.A, off, 64);
     }
     if (lane == 0 && prof.A) {
-      atomicAdd(&a.ctr->profEdges, (unsigned long long)prof.E);
-      atomicAdd(&a.ctr->profChangedEdges, (unsigned long long)prof.C);
       atomicAdd(&a.ctr->profFlagUpdates, (unsigned long long)prof.A);
       atomicAdd(&a.ctr->profFlagEdges, (unsigned long long)prof.E);
       atomicAdd(&a.ctr->profFlagChangedEdges, (unsigned long long)prof.C);
