@@ -166,6 +166,17 @@ inline bool dlp_dense_enter(long long n, int queued) {
 inline bool dlp_dense_thick(long long n, long long N) {
   return N <= (1 << 19) || n * (N <= (1 << 20) ? 64 : 16) >= N;
 }
+/* Vertices a wave of the thick walk takes at a time: its 8 groups update 8 of
+ * the flagged ones at once, one round after another, so on a small graph with
+ * a frontier that is much of it 64 leave most of the GPU idle.  us a launch,
+ * queue, 8, 16 and 64 (N, degree, frontier):
+ *     2,000, 40, 1,466   12.3  6.5  9.3  21.7    20,000, 5, 17,487   14.8  4.9  5.0  9.0
+ *     5,000, 5, 2,772     7.6  4.0  4.8   7.5    50,000, 5, 5,362     7.4  5.3  4.8  5.3
+ *     5,000, 40, 3,233   10.5  6.6  9.1  19.0    50,000, 5, 37,078   16.4  6.2  5.6  8.9
+ *     5,000, 5, 50        6.1  3.9  4.4   4.5    120,000, 7, 2,852    6.8  6.7  5.5  4.5
+ *     20,000, 5, 382      7.4  4.6  4.5   4.6    120,000, 7, 49,129  18.2 10.7  8.3  7.9
+ */
+inline int dlp_dense_span(long long N) { return N <= (1 << 14) ? 8 : (N <= (1 << 16) ? 16 : 64); }
 /* the queue of iteration k (n entries) -> flags */
 int dlp_launch_dense_enter(const PropArgs &a, int k, int N, int n, hipStream_t s);
 /* one iteration */

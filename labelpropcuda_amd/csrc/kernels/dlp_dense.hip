@@ -20,11 +20,11 @@
  * not kept up: such a vertex's stamp is at least stampBase, and the list is
  * made from the stamps once the propagation has ended (k_dense_touched).
  *
- * Measured against the queue iterations, mean of all multi-block launches of
- * a stream: 5,000 vertices 6.1 -> 4.9 us, 50,000 8.5 -> 5.2 us, 500,000
- * (frontiers of 1,000 to 250,000) 9.7 -> 6.5 us, bound by the launch and
- * three dependent round trips; 6,000,000 (frontiers of 100,000 to 450,000,
- * one vertex in 14 to 60) 101.8 -> 48.4 us, bound by the label gathers.
+ * Bound by the launch and three dependent round trips on graphs that the
+ * caches hold, by the lines of labels, flags and row places beyond (6,000,000
+ * vertices: five of six requests miss the L2s).  us a launch, queue and this,
+ * over frontiers of one vertex in ten: 5,000 vertices 6.8 and 3.9, 50,000 7.4
+ * and 4.8, 500,000 15.9 and 9.7, 6,000,000 (one in thirteen) 97.7 and 68.5.
  */
 #include <algorithm>
 
@@ -174,8 +174,9 @@ __device__ __forceinline__ void dense_fold(const PropArgs &a, int k, int lane) {
   c->updates += (unsigned long long)n;
 }
 
-/* Iteration k.  Each wave takes tiles of 64 * VPL consecutive vertices, VPL
- * flags a lane.  VPL 1 (thick frontiers): every lane loads the row place,
+/* Iteration k.  Each wave takes tiles of `span` consecutive vertices: 64 * VPL,
+ * VPL flags a lane, or fewer than 64 (dlp_dense_span).  VPL 1 (thick
+ * frontiers): every lane loads the row place,
  * label and stamp of its vertex together with its flag, so meeting a flagged
  * vertex costs no further round trip; the groups fetch them from the lanes.
  * VPL > 1 (thin ones): flags only, then the loads of the flagged vertices.
@@ -191,7 +192,7 @@ __device__ __forceinline__ void dense_fold(const PropArgs &a, int k, int lane) {
  * decision although iteration k itself writes them: it writes only when there
  * is no cycle, only the value k, and no value that large gives a cycle. */
 template <int VPL, bool WATCH>
-__global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int tiles) {
+__global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int tiles, int span) {
   __shared__ unsigned short lists[kDW][64 * VPL];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int gl = lane & (kDG - 1), grp = lane / kDG;
@@ -229,10 +230,10 @@ __global__ __launch_bounds__(kDT) void k_dense(PropArgs a, int k, int N, int til
     return;
   }
   for (int tile = gwave; tile < tiles; tile += nwaves) {  // wave-uniform
-    const int base = tile * (64 * VPL);
+    const int base = tile * span;
     if constexpr (VPL == 1) {
       const int v = base + lane;
-      const bool in = v < N;
+      const bool in = lane < span && v < N;
       const int f = in ? cur[v] : 0;
       const int stamp = in ? a.iterStamp[v] : DLP_INT_MAX;
       const float old = in ? Fold[v] : 0.0f;
@@ -460,12 +461,12 @@ int dlp_launch_dense_enter(const PropArgs &a, int k, int N, int n, hipStream_t s
 }
 
 int dlp_launch_dense(const PropArgs &a, int k, int N, bool thick, hipStream_t s) {
-  const int perTile = thick ? 64 : 64 * kDenseThinFlags;
-  const int tiles = (int)(((long long)N + perTile - 1) / perTile);
+  const int span = thick ? dlp_dense_span(N) : 64 * kDenseThinFlags;
+  const int tiles = (int)(((long long)N + span - 1) / span);
   const int blocks = dense_grid((long long)tiles * 64, kDenseMaxBlocks) + 1;
   const bool watch = a.cycles && a.mark0 && k >= kCycleFrom;
 #define DLP_LAUNCH_DENSE(V, W) \
-  hipLaunchKernelGGL((k_dense<V, W>), dim3(blocks), dim3(kDT), 0, s, a, k, N, tiles)
+  hipLaunchKernelGGL((k_dense<V, W>), dim3(blocks), dim3(kDT), 0, s, a, k, N, tiles, span)
   if (thick && watch)
     DLP_LAUNCH_DENSE(1, true);
   else if (thick)

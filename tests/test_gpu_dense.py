@@ -61,6 +61,27 @@ def test_thick_and_thin_frontiers_match_the_queue(gpu_available):
     assert runs[0][1:] == runs[1][1:]
 
 
+@pytest.mark.parametrize("n,degree", [(1 << 14, 4), ((1 << 14) + 1, 4), (1 << 16, 3),
+                                      ((1 << 16) + 1, 3), (5003, 40)])
+def test_vertices_a_wave_takes(gpu_available, n, degree):
+    """Eight vertices a wave up to 16,384, sixteen up to 65,536, 64 beyond;
+    rows of 40 entries: flagged launches against the oracle."""
+    cap = 60
+    inp = L.generate(n, degree, 5, n)
+    orc = Oracle(inp, maxIterations=cap)
+    with L.Context(inp, L.make_config(inp, maxIterations=cap)) as ctx:
+        ctx.set_tuning(localThreshold=-1)
+        ctx.set_profiling(1)
+        for b in range(inp.numBatches):
+            ctx.run_batch(b)
+            orc.run_batch(b)
+            st, ost = ctx.stats(b), orc.stats()
+            assert (st["iterations"], st["updates"]) == (ost["iterations"], ost["updates"])
+            assert np.array_equal(bits(ctx.labels()), bits(orc.labels())), f"batch {b}"
+        f = ctx.flag_profile()
+        assert f["launches"] > 100 and f["thinLaunches"] == 0
+
+
 @pytest.mark.parametrize("n,thin", [(1 << 19, False), ((1 << 19) + 1, True)])
 def test_walk_by_graph_size(gpu_available, n, thin):
     """Frontiers of a few thousand: beyond 524,288 vertices flags alone are
