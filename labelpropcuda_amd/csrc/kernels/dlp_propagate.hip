@@ -1417,11 +1417,11 @@ constexpr int kBuildRow = 8;
  * empties, k reaches maxIter, or the working set outgrows the LDS budget;
  * returns the DLP_LOCAL_* reason.  capIter is the batch's iteration cap, up
  * to which a cycle is passed over (k may then end above maxIter).  CYC:
- * queue iterations look for cycles too (dlp_cycle_skip).  The shared launch
- * of many graphs needs it, its graphs stay in queue iterations; the
- * single-graph queue kernel hands a long-lived frontier to owner mode after
- * 1,024 iterations, and the test would cost it 12 spilled registers.  All LT threads of the work-group call
- * it; `pool` is the dynamic LDS (l.ldsWords words). */
+ * queue iterations look for cycles (dlp_cycle_skip): the looking passes of the
+ * shared launch of many graphs (dlp_multi_look), whose graphs stay in queue
+ * iterations; the single-graph queue kernel hands a long-lived frontier to
+ * owner mode after 1,024.  All LT threads of the work-group call it; `pool` is
+ * the dynamic LDS (l.ldsWords words). */
 template <int LT, int SR, bool OWNER, bool MASK, bool CYC>
 __device__ __forceinline__ int local_passes(const PropArgs &a, const LocalArgs &l, int &k, int maxIter,
                             int capIter, int *pool, LocalShared &S, LocalProf &prof,
