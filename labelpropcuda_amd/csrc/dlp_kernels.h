@@ -161,10 +161,12 @@ inline bool dlp_dense_enter(long long n, int queued) {
  *                        in 25  12.0 15.8
  *   2,000,000            in 100 14.0  8.3   in 38  18.2  14.5   in 19 22.2  22.4
  *   6,000,000            in 77  36.3 17.8   in 19  56.5  52.8   in 13 70.3  68.5
- * Up to 250,000 vertices thick is never behind by more than 0.1; at 1,500,000
+ * The cycle test, from iteration 1,024 on, costs the thick walk another 4
+ * bytes a vertex (1,000,000 vertices, one in 57: 3,000 iterations 30.8 ms thick,
+ * 28.7 thin).  Up to 250,000 vertices thick is never behind by more than 0.1; at 1,500,000
  * one in 64 is too early (two streams 134 and 152 ms, against 140 and 162). */
 inline bool dlp_dense_thick(long long n, long long N) {
-  return N <= (1 << 19) || n * (N <= (1 << 20) ? 64 : 16) >= N;
+  return N <= (1 << 19) || n * (N <= (3 << 18) ? 64 : (N <= (1 << 20) ? 40 : 16)) >= N;
 }
 /* Vertices a wave of the thick walk takes at a time: its 8 groups update 8 of
  * the flagged ones at once, one round after another, so on a small graph with

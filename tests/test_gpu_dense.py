@@ -82,7 +82,7 @@ def test_vertices_a_wave_takes(gpu_available, n, degree):
         assert f["launches"] > 100 and f["thinLaunches"] == 0
 
 
-@pytest.mark.parametrize("n,thin", [(1 << 19, False), ((1 << 19) + 1, True)])
+@pytest.mark.parametrize("n,thin", [(1 << 19, False), ((1 << 19) + 1, True), ((3 << 18) + 1, True)])
 def test_walk_by_graph_size(gpu_available, n, thin):
     """Frontiers of a few thousand: beyond 524,288 vertices flags alone are
     walked, up to there every vertex's row place along with its flag."""
