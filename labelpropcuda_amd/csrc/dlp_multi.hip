@@ -275,6 +275,11 @@ class HandBackLane {
     std::lock_guard<std::mutex> lock(mu_);
     return inFlight_;
   }
+  /* graphs released so far */
+  int released() {
+    std::lock_guard<std::mutex> lock(mu_);
+    return released_;
+  }
   int workers() const { return workers_; }
   int error() {
     std::lock_guard<std::mutex> lock(mu_);
@@ -284,11 +289,11 @@ class HandBackLane {
     std::lock_guard<std::mutex> lock(mu_);
     return msg_;
   }
-  /* waits until `deadline` (seconds on `now`) or until a graph is released */
+  /* waits until `deadline` (seconds on `now`) or until a graph has been
+   * released since released() was `seen` */
   template <class Now>
-  void wait(double deadline, Now now) {
+  void wait(int seen, double deadline, Now now) {
     std::unique_lock<std::mutex> lock(mu_);
-    const int seen = released_;
     const double left = deadline - now();
     if (left <= 0) return;
     cv_.wait_for(lock, std::chrono::duration<double>(left),
@@ -1203,6 +1208,9 @@ extern "C" int dlp_multi_serve(dlp_multi *m, const dlp_serve_request *reqs, int 
   };
   while (nextArrival < numReqs || !pending.empty() || !flight.empty()) {
     if (laneFailed()) return rc;
+    /* before the graphs are looked at: one that the lane releases meanwhile
+     * may be found busy below, and the lane idle right after */
+    const int seen = lane ? lane->released() : 0;
     const double t = now();
     while (nextArrival < numReqs && reqs[nextArrival].arrival <= t) pending.push_back(nextArrival++);
     const double nextAt = nextArrival < numReqs ? reqs[nextArrival].arrival : t + 1.0;
@@ -1231,8 +1239,8 @@ extern "C" int dlp_multi_serve(dlp_multi *m, const dlp_serve_request *reqs, int 
     pending.swap(rest);
     if (flight.empty() && fresh.empty()) {
       if (pending.empty() && nextArrival >= numReqs) break;  // only hand-back work left
-      if (lane && lane->inFlight() > 0) {
-        lane->wait(nextAt, now);  // a graph or its lease comes back, or a request arrives
+      if (lane && (lane->inFlight() > 0 || lane->released() != seen)) {
+        lane->wait(seen, nextAt, now);  // a graph or its lease comes back, or a request arrives
       } else if (pending.empty()) {
         std::this_thread::sleep_for(std::chrono::duration<double>(nextAt - t));
       } else {  // cannot happen: an idle runner admits the first pending batch

@@ -130,3 +130,24 @@ def test_serving_rejects_bad_config(gpu_available, tenants):
         done, _ = m.serve([(0, 0.0)], handBackAfter=-1)  # still usable
         assert done[0] >= 0.0
 
+
+
+def test_serving_one_tenant_through_the_lane(gpu_available):
+    """Every batch leaves for the lane at its first slice stop, and the next
+    one waits for it: the runner is idle whenever the lane gives the graph
+    back, also between the looks at the two."""
+    inp = L.generate_stream(3000, 5, [0, 1500] + [40] * 60, 7)
+    cfg = L.make_config(inp, maxIterations=3000)
+    with L.Context(inp, cfg) as ctx:
+        ctx.run_all()
+        want = ctx.labels()
+    with L.Multi([inp], [cfg]) as m:
+        m.set_tuning(heavyFrontier=1 << 30)
+        for _ in range(20):
+            m.reset()
+            m.run_next([0])
+            done, _ = m.serve([(0, 0.0)] * (inp.numBatches - 1), handBackLanes=1,
+                              sliceIterations=1, sliceMs=-1.0, handBackAfter=1)
+            m.synchronize()
+            assert np.all(np.diff(done) >= 0)
+            assert np.array_equal(bits(m.labels(0)), bits(want))
